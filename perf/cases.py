@@ -251,12 +251,14 @@ _BATCH_SIZES = [(64, 64), (128, 128), (256, 144), (512, 512), (1024, 576), (1024
 
 
 def _batch_layout(case):
-    """Resolution and spp of each view, fixed by the case."""
+    """Resolution and spp of each view, fixed by the case; about 40 M paths at most."""
     g = np.random.default_rng(1000 + case["layout"])
     views, paths = [], 0
     for _ in range(case["views"]):
         w, h = _BATCH_SIZES[int(g.integers(len(_BATCH_SIZES)))]
-        spp = int(g.choice([4, 16])) if paths < 80_000_000 else 4
+        spp = int(g.choice([4, 16]))
+        if paths > 40_000_000:
+            w, h, spp = 128, 128, 4
         views.append((w, h, spp))
         paths += w * h * spp
     return views
