@@ -3,12 +3,12 @@
 // Render loop (SmallPT::run, small_pt.cpp:15-70, restructured as a wavefront): path state lives in
 // double-buffered SoA arrays in HBM. Each iteration runs
 //   raygen  -> new camera paths fill the free tail of the current buffer (Sobol + camera)
-//   closest -> closest-hit traversal of every active ray
+//   trace   -> closest-hit traversal of every active ray, and any-hit traversal of the shadow rays of the
+//              shading before; unoccluded NEE contributions are added to the path (or, for a path that
+//              ended there, to its per-sample result)
 //   shade   -> emitter/sky MIS, NEE light sample + shadow ray, BSDF sample, Russian roulette;
 //              survivors are compacted into the next buffer with a wave ballot + prefix count and
-//              one atomic per wave, shadow rays into the shadow queue the same way
-//   shadow  -> any-hit traversal; unoccluded NEE contributions are added to the path (or, for a path
-//              that ended this bounce, to its per-sample result)
+//              one atomic per block, shadow rays into the shadow queue the same way
 // and a film kernel folds the per-sample results of a batch into the FP64 film in sample order,
 // one thread per pixel, so the film is deterministic.
 #include <hip/hip_runtime.h>
@@ -249,27 +249,25 @@ __global__ __launch_bounds__(256) void k_stat_reduce(unsigned long long *stats, 
     }
 }
 
-__global__ void k_ctrl_init(Ctrl *c, uint64_t work_end) {
-    c->n_active = 0;
-    c->n_next.v = 0;
-    c->n_shadow.v = 0;
-    c->n_shadow_trace = 0;
-    c->none = 0;
-    c->iteration = 0;
-    c->work_next = 0;
-    c->work_end = work_end;
+__global__ void k_ctrl_init(Ctrl *c) {
+    for (int p = 0; p < 2; ++p) {
+        c->n_next[p].v = 0;
+        c->n_shadow[p].v = 0;
+        c->started[p] = 0;
+    }
+    for (int k = 0; k < kShadeClasses; ++k) c->n_class[k].v = 0;
 }
 
-template <bool BATCH>
-__global__ __launch_bounds__(256) void k_raygen(RenderConsts rc, PathBufs cur, const Ctrl *ctrl, uint32_t Q) {
-    uint32_t n_active = ctrl->n_active;
-    uint64_t wn = ctrl->work_next, we = ctrl->work_end;
-    uint64_t room = (uint64_t)(Q - n_active);
-    uint32_t n_gen = (uint32_t)min(room, we - wn);
-    uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n_gen) return;
-    uint32_t w = (uint32_t)(wn + t);
-    uint32_t slot = n_active + t;
+// The counts the host steers by, written to its pinned block: the state that the iteration of this parity
+// would start from.
+__global__ void k_ctrl_report(Queue q, CtrlReport *out) { *out = CtrlReport{q.kept(), q.total - q.started()}; }
+
+// New paths in the free tail of the queue.
+template <bool BATCH> __global__ __launch_bounds__(256) void k_raygen(RenderConsts rc, PathBufs cur, Queue q) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= q.fresh()) return;
+    const uint32_t w = q.started() + t;
+    const uint32_t slot = q.kept() + t;
     uint32_t x, y, s;
     uint32_t view = 0;
     if (BATCH) view = locate_batch(rc, w, x, y, s);
@@ -285,24 +283,6 @@ __global__ __launch_bounds__(256) void k_raygen(RenderConsts rc, PathBufs cur, c
     // without a read (path_beta_L)
     cur.ro[slot] = make_float4(o.x, o.y, o.z, 0.0f);
     cur.rd[slot] = make_float4(d.x, d.y, d.z, kInf);
-}
-
-// Also hands the shadow rays of the previous shading pass to this iteration's traversal (n_shadow_trace)
-// and empties the queue for this iteration's shading pass, which refills it after the traversal.
-__global__ void k_gen_done(Ctrl *c, uint32_t Q) {
-    uint64_t room = (uint64_t)(Q - c->n_active);
-    uint32_t n_gen = (uint32_t)min(room, c->work_end - c->work_next);
-    c->n_active += n_gen;
-    c->work_next += n_gen;
-    c->n_next.v = 0;
-    c->n_shadow_trace = c->n_shadow.v;
-    c->n_shadow.v = 0;
-    for (int k = 0; k < kShadeClasses; ++k) c->n_class[k].v = 0;
-}
-
-__global__ void k_iter_done(Ctrl *c) {
-    c->n_active = c->n_next.v;
-    c->iteration += 1;
 }
 
 // Closest hit for n rays (count read from *n_dev when given). Grid-stride over rays; one LDS stack
@@ -396,23 +376,33 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
     block_add_stats<kTraceBlock / 64>(stat_rows, slots, v, s_stat);
 }
 
-// One traversal launch per wavefront iteration: the closest hits of the iteration's nc rays (ro, rd -> hit)
-// and the occlusion of the ns shadow rays of the previous shading pass (sro, srd; an unoccluded ray adds
-// its contribution by add_nee). Indices [0, nc) are closest-hit queries and [nc, nc + ns) shadow rays,
-// one grid-stride sequence: the persistent grid balances both queues, and the long shadow rays of one
-// pass run beside the next pass's closest-hit rays instead of in a launch of their own, whose length
-// the slowest rays set. Node and triangle counts are kept per ray and added to the block's LDS totals of
-// the ray's kind when it ends (no per-kind registers in the loop); block 0 adds the ray counts.
+// One traversal launch per wavefront iteration: the closest hits of the iteration's nc rays (ro, rd -> hit;
+// nc is 0 with `closest` 0) and the occlusion of the ns shadow rays of the previous shading pass (sro, srd;
+// an unoccluded ray adds its contribution by add_nee). Indices [0, nc) are closest-hit queries and
+// [nc, nc + ns) shadow rays, one grid-stride sequence: the persistent grid balances both queues, and the
+// long shadow rays of one pass run beside the next pass's closest-hit rays instead of in a launch of their
+// own, whose length the slowest rays set. Node and triangle counts are kept per ray and added to the block's
+// LDS totals of the ray's kind when it ends (no per-kind registers in the loop). Block 0 adds the ray counts
+// and prepares the counters that the iteration's shading pass appends to.
 template <int W, bool ALPHA>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? 4 : 8))) void k_trace(
-    DevScene sc, const uint32_t *nc_dev, const float4 *ro, const float4 *rd, float4 *hit, const uint32_t *ns_dev,
-    const float4 *sro, const float4 *srd, const uint32_t *target, const float4 *contrib, float4 *path_L, float4 *samp,
-    float4 *recs, uint32_t *ovf, uint32_t ovf_cap, unsigned long long *stat_rows) {
+    DevScene sc, Queue q, uint32_t closest, const float4 *ro, const float4 *rd, float4 *hit, const float4 *sro,
+    const float4 *srd, const uint32_t *target, const float4 *contrib, float4 *path_L, float4 *samp, float4 *recs,
+    uint32_t *ovf, uint32_t ovf_cap, unsigned long long *stat_rows) {
     __shared__ uint32_t s_stack[kStackLds * kTraceBlock];
     __shared__ uint32_t s_cnt[5]; // closest nodes, tris; shadow nodes, tris; stack spills
-    const uint32_t nc = *nc_dev, ns = *ns_dev, n = nc + ns;
+    const uint32_t nc = closest ? q.active() : 0u, ns = q.shadows(), n = nc + ns;
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t G = gridDim.x * blockDim.x;
+    if (gid == 0) {
+        const uint32_t other = 1u - q.parity;
+        q.ctrl->n_next[other].v = 0;
+        q.ctrl->n_shadow[other].v = 0;
+        q.ctrl->started[other] = q.started() + q.fresh();
+        for (int k = 0; k < kShadeClasses; ++k) q.ctrl->n_class[k].v = 0;
+        stat_rows[kRaysClosest] += nc; // block 0's own row
+        stat_rows[kRaysShadow] += ns;
+    }
     if (blockIdx.x * blockDim.x >= n) return;
     if (threadIdx.x < 5) s_cnt[threadIdx.x] = 0u;
     __syncthreads();
@@ -460,10 +450,6 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
         row[kNodesShadow] += s_cnt[2];
         row[kTrisShadow] += s_cnt[3];
         row[kSpills] += s_cnt[4];
-        if (blockIdx.x == 0) {
-            row[kRaysClosest] += nc;
-            row[kRaysShadow] += ns;
-        }
     }
 }
 
@@ -581,10 +567,10 @@ KS_DEV float mesh_light_pdf(const DevScene &sc, const Light &l, f3 wi, float wi_
 // Material sort of the current buffer: each path's slot goes to the list of its class (a ray that left
 // the scene, or the class of the material it hit), Q entries per class, in the order of the buffer
 // within each wave.
-__global__ __launch_bounds__(256) void k_classify(DevScene sc, const float4 *hits, Ctrl *ctrl, uint32_t *order,
+__global__ __launch_bounds__(256) void k_classify(DevScene sc, const float4 *hits, Queue q, uint32_t *order,
                                                   uint32_t Q) {
     __shared__ uint32_t s_app[5];
-    const uint32_t n = ctrl->n_active;
+    const uint32_t n = q.active();
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x * blockDim.x >= n) return;
     int cls = -1;
@@ -594,7 +580,7 @@ __global__ __launch_bounds__(256) void k_classify(DevScene sc, const float4 *hit
     }
 #pragma unroll
     for (int k = 0; k < kShadeClasses; ++k) {
-        const uint32_t j = block_append<4>(&ctrl->n_class[k].v, cls == k, s_app);
+        const uint32_t j = block_append<4>(&q.ctrl->n_class[k].v, cls == k, s_app);
         if (cls == k) order[(size_t)k * Q + j] = i;
     }
 }
@@ -878,11 +864,11 @@ KS_DEV void shade_vertex(const DevScene &sc, const RenderConsts &rc, const Guide
 // whole buffer with every lobe.
 template <bool GUIDED, bool BATCH, bool TEX, int CLASS = kShadeUnsorted>
 __global__ __launch_bounds__(256) void k_shade(DevScene sc, RenderConsts rc, PathBufs cur, PathBufs nxt,
-                                               const float4 *hits, Ctrl *ctrl, float4 *sh_o, float4 *sh_d,
+                                               const float4 *hits, Queue q, float4 *sh_o, float4 *sh_d,
                                                uint32_t *sh_tgt, float4 *sh_c, float4 *samp,
                                                unsigned long long *stats, GuideShade gs, const uint32_t *order,
                                                uint32_t Q) {
-    const uint32_t n = CLASS == kShadeUnsorted ? ctrl->n_active : ctrl->n_class[CLASS].v;
+    const uint32_t n = CLASS == kShadeUnsorted ? q.active() : q.ctrl->n_class[CLASS].v;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x * blockDim.x >= n) return; // whole block idle
     const bool active = t < n;
@@ -912,8 +898,9 @@ __global__ __launch_bounds__(256) void k_shade(DevScene sc, RenderConsts rc, Pat
                                                 sh_contrib, sh_tmax, nonfinite, bounce, sob, rec_slot, view);
     }
 
-    __shared__ uint32_t s_app[5];
-    uint32_t j = block_append<4>(&ctrl->n_next.v, survive, s_app);
+    __shared__ uint32_t s_app[10];
+    uint32_t j, k;
+    block_append2<4>(&q.ctrl->n_next[1u - q.parity].v, survive, &q.ctrl->n_shadow[1u - q.parity].v, shadow, s_app, j, k);
     if (survive) {
         nxt.work[j] = w;
         nxt.state[j] = (uint32_t)sob.dim | ((uint32_t)(bounce + 1) << 16);
@@ -922,7 +909,6 @@ __global__ __launch_bounds__(256) void k_shade(DevScene sc, RenderConsts rc, Pat
         nxt.ro[j] = make_float4(new_o.x, new_o.y, new_o.z, 0.0f);
         nxt.rd[j] = make_float4(new_d.x, new_d.y, new_d.z, kInf);
     }
-    uint32_t k = block_append<4>(&ctrl->n_shadow.v, shadow, s_app);
     if (shadow) {
         sh_o[k] = make_float4(sh_origin.x, sh_origin.y, sh_origin.z, 0.0f);
         sh_d[k] = make_float4(sh_dir.x, sh_dir.y, sh_dir.z, sh_tmax);
@@ -941,12 +927,11 @@ __global__ __launch_bounds__(256) void k_shade(DevScene sc, RenderConsts rc, Pat
 // single addition the wavefront's traversal makes (add_nee). Plain renders of scenes without alpha-tested
 // triangles only; n paths of buffer cur, n no larger than the overflow area's lanes.
 template <int W, bool BATCH, bool TEX>
-__global__ __launch_bounds__(256) void k_tail(DevScene sc, RenderConsts rc, PathBufs cur, const uint32_t *n_dev,
-                                              float4 *samp, uint32_t *ovf, uint32_t ovf_cap,
-                                              unsigned long long *stat_rows) {
+__global__ __launch_bounds__(256) void k_tail(DevScene sc, RenderConsts rc, PathBufs cur, Queue q, float4 *samp,
+                                              uint32_t *ovf, uint32_t ovf_cap, unsigned long long *stat_rows) {
     __shared__ uint32_t s_stack[kStackLds * 256];
     __shared__ uint32_t s_stat[3 * 4];
-    const uint32_t n = *n_dev;
+    const uint32_t n = q.active();
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x * blockDim.x >= n) return; // whole block idle
     uint32_t n_rays = 0, nonfinite = 0, spills = 0;
@@ -1424,7 +1409,7 @@ struct ks_device {
     uint64_t tune_items = 0;
     uint32_t tune_q = 0;
     int tune_bpc = 0;
-    Ctrl *host_ctrl = nullptr; // pinned
+    CtrlReport *host_ctrl = nullptr; // pinned, written by k_ctrl_report
     uint8_t *host_scratch = nullptr; // pinned, 64 bytes
     double *relmse_scratch = nullptr; // this device's address of `scratch` (hipGetSymbolAddress at open)
     DevBuf perm_tab; // the sampler's permutation bytes (kPermTabDims x kPermTabPrefixes), filled at open
@@ -1760,68 +1745,83 @@ struct WavefrontOpts {
 // With opts.graph, two iterations (buffer 0 -> 1 and 1 -> 0) are captured once into a HIP graph and the
 // graph is replayed; the kernels read their counts from the control block, so every replay is valid.
 // Ray capture: append the n rays of a queue after the *count already captured, up to cap rays.
-__global__ __launch_bounds__(256) void k_capture(const uint32_t *n, const float4 *ro, const float4 *rd, float4 *out,
-                                                 const uint32_t *count, uint32_t cap) {
+// shadow 1 takes the shadow rays that the iteration traces, 0 its closest-hit rays.
+__global__ __launch_bounds__(256) void k_capture(Queue q, uint32_t shadow, const float4 *ro, const float4 *rd,
+                                                 float4 *out, const uint32_t *count, uint32_t cap) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t base = *count;
-    if (i < *n && base + (uint64_t)i < cap) {
+    if (i < (shadow ? q.shadows() : q.active()) && base + (uint64_t)i < cap) {
         out[2 * (size_t)(base + i)] = ro[i];
         out[2 * (size_t)(base + i) + 1] = rd[i];
     }
 }
-__global__ void k_capture_done(const uint32_t *n, uint32_t *count, uint32_t cap) {
-    *count = (uint32_t)min((uint64_t)cap, (uint64_t)*count + *n);
+__global__ void k_capture_done(Queue q, uint32_t shadow, uint32_t *count, uint32_t cap) {
+    *count = (uint32_t)min((uint64_t)cap, (uint64_t)*count + (shadow ? q.shadows() : q.active()));
 }
 
-int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, Timer &tm, ks_render_stats *stats,
-                  const GuidePass *gp = nullptr, const WavefrontOpts &wo = WavefrontOpts{}) {
+int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int max_bounces, Timer &tm,
+                  ks_render_stats *stats, const GuidePass *gp = nullptr, const WavefrontOpts &wo = WavefrontOpts{}) {
     ks_device *dev = sc->dev;
     Workspace &ws = dev->ws;
     hipStream_t s = dev->stream;
-    Ctrl *ctrl = ws.ctrl.as<Ctrl>();
     unsigned long long *st = ws.stats.as<unsigned long long>();
-    hipLaunchKernelGGL(k_ctrl_init, dim3(1), dim3(1), 0, s, ctrl, (uint64_t)total);
+    const bool sorted = dev->sorted_shading && !sc->ds.textured;
+    Ctrl *ctrl = ws.ctrl.as<Ctrl>();
+    auto view = [&](int parity) { return Queue{ctrl, (uint32_t)parity, Q, (uint32_t)total}; };
+    hipLaunchKernelGGL(k_ctrl_init, dim3(1), dim3(1), 0, s, ctrl);
     KS_HIP(hipGetLastError());
     PathBufs pb[2];
     for (int b = 0; b < 2; ++b)
         pb[b] = PathBufs{ws.work[b].as<uint32_t>(), ws.state[b].as<uint32_t>(), ws.beta[b].as<float4>(),
                          ws.L[b].as<float4>(),     ws.ro[b].as<float4>(),     ws.rd[b].as<float4>()};
     const int tblocks = (int)((Q + 255) / 256);
-    // Blocks of ray generation and shading: one thread per queue slot until a control read bounds the
-    // work left. From a read on, an iteration holds at most the paths then active plus the work items not
-    // yet started, and generates at most the latter, so the late iterations' launches stay small.
-    int gen_blocks = tblocks, shade_blocks = tblocks;
-    const int tgrid = trace_grid(dev, sc->ds, Q, wo.blocks_per_cu);
+    // Blocks of ray generation and shading: one thread per path slot until a control read bounds the work
+    // left. From a read on, an iteration holds at most the paths then live plus the work items not yet
+    // started, and generates at most the latter, so the late iterations' launches stay small (no work left:
+    // no ray generation at all). The traversal's persistent grid is bounded the same way; its shadow rays
+    // come from the iteration before, which the previous bound covers.
+    int gen_blocks = tblocks, shade_blocks = tblocks, shade_blocks_before = tblocks;
+    auto trace_blocks = [&] {
+        return trace_grid(dev, sc->ds, (uint32_t)(shade_blocks + shade_blocks_before) * 256u, wo.blocks_per_cu);
+    };
     const bool graph = wo.graph && !gp;
+    auto launch_rays = [&](int cur, uint32_t closest) {
+        launch_trace(sc->ds, dim3(trace_blocks()), s, view(cur), closest, (const float4 *)pb[cur].ro,
+                     (const float4 *)pb[cur].rd, ws.hit.as<float4>(), (const float4 *)ws.sh_o.as<float4>(),
+                     (const float4 *)ws.sh_d.as<float4>(), (const uint32_t *)ws.sh_tgt.as<uint32_t>(),
+                     (const float4 *)ws.sh_c.as<float4>(), pb[cur].L, ws.samp.as<float4>(),
+                     gp ? gp->shade.recs : (float4 *)nullptr, ws.ovf.as<uint32_t>(), ws.ovf_cap, stat_rows(dev));
+    };
     // One iteration reading buffer cur and writing buffer 1 - cur; no events while a graph is captured.
     // Its traversal also traces the previous shading pass's shadow rays (k_trace): their contributions go
-    // to the survivors' slots [0, n_next) of buffer cur (ray generation fills the slots after them) and to
-    // per-sample results, before this iteration's shading reads the slots and refills the shadow queue.
+    // to the survivors' slots of buffer cur (ray generation fills the slots after them) and to per-sample
+    // results, before this iteration's shading reads the slots and refills the shadow queue.
     // Guide inference serves only vertices below the guide's max bounce. A path generated in iteration g
     // is at bounce i - g in iteration i, so once every work item has started by iteration last_gen (known
     // from the start when the queue holds the whole pass, else from a control read), iterations at or
     // beyond last_gen + max bounce have no guided vertex and skip the inference.
     int iter_index = 0;
     int last_gen = total <= (uint64_t)Q ? 0 : -1; // -1: not known yet
+    bool capturing = false;
     auto iteration = [&](int cur) -> int {
-        hipEvent_t e = graph ? nullptr : tm.begin(KS_K_RAYGEN);
-        if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[cur], ctrl, Q);
-        else hipLaunchKernelGGL(k_raygen<false>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[cur], ctrl, Q);
-        hipLaunchKernelGGL(k_gen_done, dim3(1), dim3(1), 0, s, ctrl, Q);
-        tm.end(e);
-        if (wo.cap_n) {
-            hipLaunchKernelGGL(k_capture, dim3(tblocks), dim3(256), 0, s, (const uint32_t *)&ctrl->n_active,
-                               (const float4 *)pb[cur].ro, (const float4 *)pb[cur].rd, wo.cap_c, wo.cap_n, wo.cap_max);
-            hipLaunchKernelGGL(k_capture_done, dim3(1), dim3(1), 0, s, (const uint32_t *)&ctrl->n_active, wo.cap_n,
-                               wo.cap_max);
+        const Queue q = view(cur);
+        hipEvent_t e = nullptr;
+        if (gen_blocks > 0) {
+            e = capturing ? nullptr : tm.begin(KS_K_RAYGEN);
+            if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[cur], q);
+            else hipLaunchKernelGGL(k_raygen<false>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[cur], q);
+            tm.end(e);
         }
-        e = graph ? nullptr : tm.begin(KS_K_CLOSEST);
-        launch_trace(sc->ds, dim3(tgrid), s, (const uint32_t *)&ctrl->n_active, (const float4 *)pb[cur].ro,
-                     (const float4 *)pb[cur].rd, ws.hit.as<float4>(), (const uint32_t *)&ctrl->n_shadow_trace,
-                     (const float4 *)ws.sh_o.as<float4>(), (const float4 *)ws.sh_d.as<float4>(),
-                     (const uint32_t *)ws.sh_tgt.as<uint32_t>(), (const float4 *)ws.sh_c.as<float4>(), pb[cur].L,
-                     ws.samp.as<float4>(), gp ? gp->shade.recs : (float4 *)nullptr, ws.ovf.as<uint32_t>(), ws.ovf_cap,
-                     stat_rows(dev));
+        if (wo.cap_n) {
+            hipLaunchKernelGGL(k_capture, dim3(tblocks), dim3(256), 0, s, q, 0u, (const float4 *)pb[cur].ro,
+                               (const float4 *)pb[cur].rd, wo.cap_c, wo.cap_n, wo.cap_max);
+            hipLaunchKernelGGL(k_capture_done, dim3(1), dim3(1), 0, s, q, 0u, wo.cap_n, wo.cap_max);
+            hipLaunchKernelGGL(k_capture, dim3(tblocks), dim3(256), 0, s, q, 1u, (const float4 *)ws.sh_o.as<float4>(),
+                               (const float4 *)ws.sh_d.as<float4>(), wo.cap_s, wo.cap_n + 1, wo.cap_max);
+            hipLaunchKernelGGL(k_capture_done, dim3(1), dim3(1), 0, s, q, 1u, wo.cap_n + 1, wo.cap_max);
+        }
+        e = capturing ? nullptr : tm.begin(KS_K_CLOSEST);
+        launch_rays(cur, 1u);
         tm.end(e);
         auto young = [&](int b) { return last_gen < 0 || iter_index - last_gen < b; };
         const bool guided_vertices = gp && young(gp->shade.max_bounce);
@@ -1831,43 +1831,33 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, Tim
         if (gp && gp->shade.mix && guided_vertices) {
             e = tm.begin(KS_K_GUIDE);
             // the guided queries are among the paths shading takes: the same launch bound holds
-            const uint32_t n_max = (uint32_t)std::min<uint64_t>(Q, (uint64_t)shade_blocks * 256u);
-            int ge = ksg::launch_infer(gp->guide, sc->ds, &ctrl->n_active, n_max, pb[cur].rd, ws.hit.as<float4>(),
+            int ge = ksg::launch_infer(gp->guide, sc->ds, q, (uint32_t)shade_blocks, pb[cur].rd, ws.hit.as<float4>(),
                                        pb[cur].state, gp->shade.max_bounce, gp->mix, gp->list, gp->n_list, s);
             tm.end(e);
             if (ge) return ge;
         }
-        e = graph ? nullptr : tm.begin(KS_K_SHADE);
-        const bool sorted = dev->sorted_shading && !sc->ds.textured;
+        e = capturing ? nullptr : tm.begin(KS_K_SHADE);
         if (sorted)
-            hipLaunchKernelGGL(k_classify, dim3(tblocks), dim3(256), 0, s, sc->ds, (const float4 *)ws.hit.as<float4>(),
-                               ctrl, ws.order.as<uint32_t>(), Q);
+            hipLaunchKernelGGL(k_classify, dim3(tblocks), dim3(256), 0, s, sc->ds, (const float4 *)ws.hit.as<float4>(), q,
+                               ws.order.as<uint32_t>(), Q);
         launch_shade(sc->ds.textured != 0, guided_shade, wo.batch, sorted, dim3(shade_blocks), s, sc->ds, rc, pb[cur],
-                     pb[1 - cur], ws.hit.as<float4>(), ctrl, ws.sh_o.as<float4>(), ws.sh_d.as<float4>(),
+                     pb[1 - cur], ws.hit.as<float4>(), q, ws.sh_o.as<float4>(), ws.sh_d.as<float4>(),
                      ws.sh_tgt.as<uint32_t>(), ws.sh_c.as<float4>(), ws.samp.as<float4>(), st,
                      gp ? gp->shade : GuideShade{}, (const uint32_t *)ws.order.as<uint32_t>(), Q);
         tm.end(e);
-        if (wo.cap_n) {
-            hipLaunchKernelGGL(k_capture, dim3(tblocks), dim3(256), 0, s, (const uint32_t *)&ctrl->n_shadow.v,
-                               (const float4 *)ws.sh_o.as<float4>(), (const float4 *)ws.sh_d.as<float4>(), wo.cap_s,
-                               wo.cap_n + 1, wo.cap_max);
-            hipLaunchKernelGGL(k_capture_done, dim3(1), dim3(1), 0, s, (const uint32_t *)&ctrl->n_shadow.v, wo.cap_n + 1,
-                               wo.cap_max);
-        }
-        hipLaunchKernelGGL(k_iter_done, dim3(1), dim3(1), 0, s, ctrl);
         return KS_OK;
     };
     // The last shading pass's shadow rays: a traversal of them alone, once the loop has ended (or before
     // the tail kernel takes the remaining paths).
     auto flush_shadow = [&](int cur) -> int {
-        hipLaunchKernelGGL(k_gen_done, dim3(1), dim3(1), 0, s, ctrl, Q); // no work left: only moves the queue
+        if (wo.cap_n) {
+            const Queue q = view(cur);
+            hipLaunchKernelGGL(k_capture, dim3(tblocks), dim3(256), 0, s, q, 1u, (const float4 *)ws.sh_o.as<float4>(),
+                               (const float4 *)ws.sh_d.as<float4>(), wo.cap_s, wo.cap_n + 1, wo.cap_max);
+            hipLaunchKernelGGL(k_capture_done, dim3(1), dim3(1), 0, s, q, 1u, wo.cap_n + 1, wo.cap_max);
+        }
         hipEvent_t e = tm.begin(KS_K_SHADOW);
-        launch_trace(sc->ds, dim3(tgrid), s, (const uint32_t *)&ctrl->none, (const float4 *)pb[cur].ro,
-                     (const float4 *)pb[cur].rd, ws.hit.as<float4>(), (const uint32_t *)&ctrl->n_shadow_trace,
-                     (const float4 *)ws.sh_o.as<float4>(), (const float4 *)ws.sh_d.as<float4>(),
-                     (const uint32_t *)ws.sh_tgt.as<uint32_t>(), (const float4 *)ws.sh_c.as<float4>(), pb[cur].L,
-                     ws.samp.as<float4>(), gp ? gp->shade.recs : (float4 *)nullptr, ws.ovf.as<uint32_t>(), ws.ovf_cap,
-                     stat_rows(dev));
+        launch_rays(cur, 0u);
         tm.end(e);
         KS_HIP(hipGetLastError());
         return KS_OK;
@@ -1876,8 +1866,10 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, Tim
     hipGraph_t g = nullptr;
     if (graph) {
         KS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        capturing = true;
         int e0 = iteration(0);
         int e1 = iteration(1);
+        capturing = false;
         hipError_t ce = hipStreamEndCapture(s, &g);
         if (e0 || e1) {
             if (g) (void)hipGraphDestroy(g);
@@ -1894,6 +1886,9 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, Tim
     int iterations = 0;
     const int check_every = 8; // empty trailing iterations cost only launch latency
     int status = KS_OK;
+    // A path generated in iteration g has ended after iteration g + max_bounces: once every work item has
+    // started by last_gen, the loop needs no control read to know its end.
+    auto all_done = [&] { return last_gen >= 0 && iterations > last_gen + max_bounces; };
     // The tail: once every work item has started and at most tail_limit paths remain, one k_tail launch
     // carries them to their ends (eager plain renders of scenes without alpha-tested triangles; not while
     // rays are captured). The control block is read after every iteration from the first read that finds
@@ -1901,8 +1896,9 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, Tim
     const uint32_t tail_limit = std::min<uint32_t>(dev->tail_paths, ws.ovf_grid);
     const bool tail_ok = !graph && !gp && !wo.cap_n && !sc->ds.alpha && tail_limit > 0;
     bool check_each = tail_ok && total <= (uint64_t)Q * check_every, tail_ran = false;
-    while (true) {
-        if (graph) {
+    bool replay = graph; // the graph's launches are as large as the queue: it serves while the queue is full
+    while (!all_done()) {
+        if (replay) {
             hipError_t le = hipGraphLaunch(exec, s);
             if (le != hipSuccess) {
                 ksa::set_error(std::string("hipGraphLaunch failed: ") + hipGetErrorString(le));
@@ -1921,36 +1917,37 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, Tim
             }
             cur = 1 - cur;
             ++iterations;
-            iter_index = iterations;
+            shade_blocks_before = shade_blocks;
         }
+        iter_index = iterations;
+        if (all_done()) break;
         // the control block is also read after iterations 1, 2 and 4, so that the launch bounds tighten early
-        const bool early_read = !graph && (iterations == 1 || iterations == 2 || iterations == 4);
+        const bool early_read = iterations == 1 || iterations == 2 || iterations == 4;
         if (iterations % check_every == 0 || check_each || early_read) {
-            hipError_t me = hipMemcpyAsync(dev->host_ctrl, ctrl, sizeof(Ctrl), hipMemcpyDeviceToHost, s);
+            hipLaunchKernelGGL(k_ctrl_report, dim3(1), dim3(64), 0, s, view(cur), dev->host_ctrl);
+            hipError_t me = hipGetLastError();
             if (me == hipSuccess) me = hipStreamSynchronize(s);
             if (me != hipSuccess) {
                 ksa::set_error(std::string("wavefront control read failed: ") + hipGetErrorString(me));
                 status = KS_ERR_HIP;
                 break;
             }
-            const uint32_t n_left = dev->host_ctrl->n_active;
-            if (n_left == 0 && dev->host_ctrl->work_next >= dev->host_ctrl->work_end) break;
-            if (last_gen < 0 && dev->host_ctrl->work_next >= dev->host_ctrl->work_end) last_gen = iterations - 1;
-            if (!graph) {
-                const uint64_t todo = dev->host_ctrl->work_end - dev->host_ctrl->work_next;
-                gen_blocks = (int)std::max<uint64_t>(1, std::min<uint64_t>(tblocks, (todo + 255) / 256));
-                shade_blocks = (int)std::max<uint64_t>(1, std::min<uint64_t>(tblocks, (n_left + todo + 255) / 256));
-            }
-            if (tail_ok && dev->host_ctrl->work_end - dev->host_ctrl->work_next <= (uint64_t)Q * check_every)
-                check_each = true;
-            if (tail_ok && dev->host_ctrl->work_next >= dev->host_ctrl->work_end) {
-                if (n_left <= tail_limit) {
+            const CtrlReport c = *dev->host_ctrl;
+            if (c.paths == 0 && c.todo == 0) break;
+            if (last_gen < 0 && c.todo == 0) last_gen = iterations - 1;
+            const uint64_t held = (uint64_t)c.paths + c.todo;
+            gen_blocks = (int)std::min<uint64_t>(tblocks, ((uint64_t)c.todo + 255) / 256);
+            shade_blocks = (int)std::max<uint64_t>(1, std::min<uint64_t>(tblocks, (held + 255) / 256));
+            // eager launches of the size of the work left from here on, once that is half the queue
+            if (replay && 2 * shade_blocks <= tblocks) replay = false;
+            if (tail_ok && c.todo <= (uint64_t)Q * check_every) check_each = true;
+            if (tail_ok && c.todo == 0) {
+                if (c.paths <= tail_limit) {
                     status = flush_shadow(cur); // the last shading pass's shadow rays add to these paths
                     if (status) break;
                     hipEvent_t e = tm.begin(KS_K_TAIL);
-                    launch_tail(sc->ds, wo.batch, dim3((n_left + 255) / 256), s, rc, pb[cur],
-                                (const uint32_t *)&ctrl->n_active, ws.samp.as<float4>(), ws.ovf.as<uint32_t>(),
-                                ws.ovf_cap, stat_rows(dev));
+                    launch_tail(sc->ds, wo.batch, dim3((unsigned)((c.paths + 255) / 256)), s, rc, pb[cur], view(cur),
+                                ws.samp.as<float4>(), ws.ovf.as<uint32_t>(), ws.ovf_cap, stat_rows(dev));
                     tm.end(e);
                     KS_HIP(hipGetLastError());
                     tail_ran = true;
@@ -1964,7 +1961,7 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, Tim
             }
         }
     }
-    if (status == KS_OK && !tail_ran) status = flush_shadow(graph ? 0 : cur);
+    if (status == KS_OK && !tail_ran) status = flush_shadow(cur);
     if (exec) (void)hipGraphExecDestroy(exec);
     if (g) (void)hipGraphDestroy(g);
     if (status) return status;
@@ -2057,7 +2054,7 @@ int ks_device_open(int32_t ordinal, ks_device **out) {
         hipDeviceProp_t prop;
         KS_HIP(hipGetDeviceProperties(&prop, ordinal));
         d->n_cu = prop.multiProcessorCount;
-        KS_HIP(hipHostMalloc((void **)&d->host_ctrl, sizeof(Ctrl), hipHostMallocDefault));
+        KS_HIP(hipHostMalloc((void **)&d->host_ctrl, sizeof(CtrlReport), hipHostMallocDefault));
         KS_HIP(hipHostMalloc((void **)&d->host_scratch, 64, hipHostMallocDefault));
         // the allocation-free relMSE's scratch: its address on this device (the current one)
         void *sp = nullptr;
@@ -2964,7 +2961,7 @@ int ks_small_pt_render(ks_scene *scene, const ks_camera_desc *cam, const ks_smal
                 rc.nb = std::min(spp_chunk, s_end - c0);
                 rc.work_list = nullptr;
                 uint64_t total = pixels * (uint64_t)rc.nb;
-                e = run_wavefront(scene, rc, total, Q, tm, stats);
+                e = run_wavefront(scene, rc, total, Q, rc.bounces, tm, stats);
                 if (e) return e;
                 hipEvent_t ev = tm.begin(KS_K_FILM);
                 hipLaunchKernelGGL(k_film, dim3((unsigned)((pixels + 255) / 256)), dim3(256), 0, dev->stream, rc,
@@ -3120,7 +3117,7 @@ int ks_small_pt_render_guided(ks_scene *scene, const ks_camera_desc *cam, const 
                 gw.stamp = 0;
             }
             gp.shade.stamp = ++gw.stamp;
-            e = run_wavefront(scene, rc, pixels * (uint64_t)nb, Q, tm, stats, &gp);
+            e = run_wavefront(scene, rc, pixels * (uint64_t)nb, Q, rc.bounces, tm, stats, &gp);
             if (e) return e;
             hipEvent_t ev = tm.begin(KS_K_FILM);
             hipLaunchKernelGGL(k_film, dim3((unsigned)((pixels + 255) / 256)), dim3(256), 0, dev->stream, rc,
@@ -3238,6 +3235,7 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
         std::vector<int> spp((size_t)n_views);
         std::vector<double *> rgbs((size_t)n_views), wtss((size_t)n_views);
         uint64_t paths = 0, max_pixels = 0;
+        int max_bounces = 0;
         for (int v = 0; v < n_views; ++v) {
             const ks_batch_view &bv = views[v];
             KS_REQUIRE(bv.film && bv.film->dev == dev, "every view needs a film on the scene's device");
@@ -3246,6 +3244,7 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
             int e = fill_consts(scene->dev, scene, &bv.camera, &bv.params, hv[v]);
             if (e) return e;
             spp[v] = bv.params.spp;
+            max_bounces = std::max(max_bounces, hv[v].bounces);
             rgbs[v] = bv.film->rgb.as<double>();
             wtss[v] = bv.film->wts.as<double>();
             uint64_t P = (uint64_t)hv[v].cw * hv[v].ch;
@@ -3309,7 +3308,7 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
                     int saved = dev->timing;
                     dev->timing = 0;
                     KS_HIP(hipEventRecord(ea, dev->stream));
-                    e = run_wavefront(scene, prc, probe.items, q, ptm, nullptr, nullptr, pw);
+                    e = run_wavefront(scene, prc, probe.items, q, max_bounces, ptm, nullptr, nullptr, pw);
                     KS_HIP(hipEventRecord(eb, dev->stream));
                     dev->timing = saved;
                     if (e) return e;
@@ -3348,7 +3347,7 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
             rc.views = dviews.p();
             rc.segs = dsegs.p();
             rc.n_segs = (int32_t)c.segs.size();
-            e = run_wavefront(scene, rc, c.items, Q, tm, stats, nullptr, wo);
+            e = run_wavefront(scene, rc, c.items, Q, max_bounces, tm, stats, nullptr, wo);
             if (e) return e;
             hipEvent_t ev = tm.begin(KS_K_FILM);
             hipLaunchKernelGGL(k_film_batch, dim3((c.threads + 255) / 256), dim3(256), 0, dev->stream, dviews.p(), dsegs.p(),
@@ -3398,7 +3397,7 @@ int ks_trace_samples(ks_scene *scene, const ks_camera_desc *cam, const ks_small_
         if (e) return e;
         clear_stats(dev, dev->stream);
         Timer tm{dev};
-        e = run_wavefront(scene, rc, (uint64_t)n, Q, tm, nullptr);
+        e = run_wavefront(scene, rc, (uint64_t)n, Q, rc.bounces, tm, nullptr);
         if (e) return e;
         tm.collect(nullptr);
         std::vector<float4> res((size_t)n);
@@ -3453,7 +3452,7 @@ int ks_trace_capture(ks_scene *scene, const ks_camera_desc *cam, const ks_small_
         wo.cap_n = cn.as<uint32_t>();
         wo.cap_max = (uint32_t)max_rays;
         Timer tm{dev};
-        e = run_wavefront(scene, rc, (uint64_t)n, Q, tm, nullptr, nullptr, wo);
+        e = run_wavefront(scene, rc, (uint64_t)n, Q, rc.bounces, tm, nullptr, nullptr, wo);
         if (e) return e;
         tm.collect(nullptr);
         uint32_t counts[2];

@@ -151,20 +151,12 @@ struct QueryArray { // queries n x 9: position, normal, wo
 
 struct QueryHits { // wavefront paths with a surface hit: position, geometric normal facing wo, wo
     DevScene sc;
-    const uint32_t *n_dev;
     const float4 *rd;
     const float4 *hits;
     const uint32_t *state; // path state: bounce in bits 16..23
     int32_t max_bounce;    // paths at this bounce or deeper are not guided: no query
-    __device__ uint32_t count() const { return *n_dev; }
-    __device__ uint32_t slot(uint32_t i) const { return i; }
     __device__ bool wanted(uint32_t i) const {
         return (int32_t)((state[i] >> 16) & 0xffu) < max_bounce && __float_as_int(hits[i].w) >= 0;
-    }
-    __device__ bool load(uint32_t i, f3 &p, f3 &nn, f3 &wo) const {
-        if (i >= *n_dev) return false;
-        if ((int32_t)((state[i] >> 16) & 0xffu) >= max_bounce) return false;
-        return load_slot(i, p, nn, wo);
     }
     __device__ bool load_slot(uint32_t i, f3 &p, f3 &nn, f3 &wo) const {
         float4 h = hits[i];
@@ -193,9 +185,9 @@ struct QueryList {
     }
 };
 
-__global__ __launch_bounds__(256) void k_guide_compact(QueryHits h, uint32_t *list, uint32_t *n_list) {
+__global__ __launch_bounds__(256) void k_guide_compact(QueryHits h, Queue q, uint32_t *list, uint32_t *n_list) {
     __shared__ uint32_t s_app[5];
-    const uint32_t n = *h.n_dev;
+    const uint32_t n = q.active();
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x * blockDim.x >= n) return;
     const bool want = i < n && h.wanted(i);
@@ -964,13 +956,13 @@ int32_t guide_batch(const ks_guide *g) { return g->cfg.train_batch; }
 int32_t guide_max_steps(const ks_guide *g) { return g->cfg.max_steps_per_pass; }
 int32_t guide_train_spp(const ks_guide *g) { return g->cfg.train_spp; }
 
-int launch_infer(ks_guide *g, const DevScene &sc, const uint32_t *n_dev, uint32_t n_max, const float4 *rd,
+int launch_infer(ks_guide *g, const DevScene &sc, const Queue &q, uint32_t blocks, const float4 *rd,
                  const float4 *hits, const uint32_t *state, int32_t max_bounce, float4 *mix, uint32_t *list,
                  uint32_t *n_list, hipStream_t s) {
-    unsigned blocks = (n_max + kInferBlock - 1) / kInferBlock;
-    const QueryHits qh{sc, n_dev, rd, hits, state, max_bounce};
+    const QueryHits qh{sc, rd, hits, state, max_bounce};
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, n_list);
-    hipLaunchKernelGGL(k_guide_compact, dim3((n_max + 255) / 256), dim3(256), 0, s, qh, list, n_list);
+    hipLaunchKernelGGL(k_guide_compact, dim3(blocks), dim3(256), 0, s, qh, q, list, n_list);
+    static_assert(kInferBlock == 256, "the inference launch covers as many queries as the shading launch");
     const QueryList ql{qh, list, n_list};
     if (g->fp8)
         hipLaunchKernelGGL((k_guide_infer<QueryList, 2>), dim3(blocks), dim3(kInferBlock), 0, s, net_of(g), ql, mix,

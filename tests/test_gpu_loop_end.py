@@ -1,0 +1,34 @@
+"""The wavefront loop's end: known from the bounce count where the queue holds the whole pass, read from the
+control block otherwise, and a batch that leaves graph replay for bounded launches. Every path must be
+carried to its end in each, so the films are equal bit for bit."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bounces", [0, 1, 2, 7, 8, 17])
+@pytest.mark.parametrize("size,spp", [((3, 1), 1), ((31, 17), 3), ((64, 48), 4)])
+def test_known_and_read_ends_agree(ks, device, cornell, bounces, size, spp):
+    print("loop end", bounces, size, spp, flush=True)
+    sc = ks.Scene(device, cornell)
+    w, h = size
+    out = []
+    # the queue that holds every path; one that refills (at least 256 slots); batches, replayed and eager
+    for queue, batch, graph in ((0, False, False), (256, False, False), (256, True, True), (4096, True, True),
+                                (0x10000, True, False)):
+        film = ks.Film(device, w, h)
+        p = ks.small_pt_params(bounces=bounces, render_width=w, render_height=h, spp=spp, spp_prog_interval=spp,
+                               rng_seed=7, queue_size=queue)
+        if batch:
+            st = ks.small_pt_render_batch(sc, [(cornell.camera, p, film)], queue_size=queue, graph=graph)
+        else:
+            st = ks.small_pt_render(sc, cornell.camera, p, film)
+        out.append((film.download(), st["rays_closest"], st["rays_shadow"]))
+        film.close()
+    sc.close()
+    (rgb, wts), rc, rs = out[0]
+    assert wts.sum() == w * h * spp
+    for (r, g), c, s in out[1:]:
+        assert np.array_equal(r, rgb) and np.array_equal(g, wts) and (c, s) == (rc, rs)
