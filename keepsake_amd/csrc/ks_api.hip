@@ -862,8 +862,12 @@ KS_DEV void shade_vertex(const DevScene &sc, const RenderConsts &rc, const Guide
 // per class) and is compiled for that class only: kShadeMiss holds only the escaped-ray code, the
 // dielectric and metal classes the BSDF lobes their materials can weight. kShadeUnsorted shades the
 // whole buffer with every lobe.
+// Bound by its VALU instructions (1.04 a cycle and CU on the 720p room, 4800 per wave of path vertices before
+// the sampler's digit table, about 4000 with it). The plain kernels are held to 96 VGPRs, 5 waves per SIMD;
+// left alone they take 98 (103 batched) and run at 4.
 template <bool GUIDED, bool BATCH, bool TEX, int CLASS = kShadeUnsorted>
-__global__ __launch_bounds__(256) void k_shade(DevScene sc, RenderConsts rc, PathBufs cur, PathBufs nxt,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(!GUIDED && !TEX && CLASS == kShadeUnsorted ? 5 : 2)))
+void k_shade(DevScene sc, RenderConsts rc, PathBufs cur, PathBufs nxt,
                                                const float4 *hits, Queue q, float4 *sh_o, float4 *sh_d,
                                                uint32_t *sh_tgt, float4 *sh_c, float4 *samp,
                                                unsigned long long *stats, GuideShade gs, const uint32_t *order,
@@ -1152,15 +1156,14 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double *partials, un
 
 // The sampler's permutation table: one thread per (dimension, digit prefix) entry, kPermTabDims x
 // kPermTabPrefixes threads in all.
-__global__ __launch_bounds__(256) void k_perm_tab(uint8_t *tab) {
+__global__ __launch_bounds__(256) void k_perm_tab(uint32_t *tab) {
     const uint32_t e = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t dim = e / kPermTabPrefixes, h = e % kPermTabPrefixes;
-    tab[e] = (uint8_t)perm4_byte(perm_index(h ^ (0x55555555u * dim)));
+    tab[e] = perm_tab_entry(e / kPermTabPrefixes, e % kPermTabPrefixes);
 }
 
 __global__ void k_sobol_stream(int64_t n, const int32_t *px, const int32_t *py, const int32_t *sample, int32_t seed,
                                int32_t log2spp, int32_t ndigits, int32_t n_calls, const int32_t *kinds,
-                               int32_t n_values, const uint8_t *perm_tab, uint32_t *out_u32, float *out_f) {
+                               int32_t n_values, const uint32_t *perm_tab, uint32_t *out_u32, float *out_f) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     Sobol sob;
@@ -1412,7 +1415,7 @@ struct ks_device {
     CtrlReport *host_ctrl = nullptr; // pinned, written by k_ctrl_report
     uint8_t *host_scratch = nullptr; // pinned, 64 bytes
     double *relmse_scratch = nullptr; // this device's address of `scratch` (hipGetSymbolAddress at open)
-    DevBuf perm_tab; // the sampler's permutation bytes (kPermTabDims x kPermTabPrefixes), filled at open
+    DevBuf perm_tab; // the sampler's permuted digits (kPermTabDims x kPermTabPrefixes words), filled at open
     int sorted_shading = 0;           // material-sorted shading of untextured scenes (ks_device_set_shading)
     uint32_t tail_paths = 0;          // k_tail takes over at or below this many paths (ks_device_set_tail; 0: off)
     std::vector<hipEvent_t> events; // timing event pool, reused across renders
@@ -1703,7 +1706,7 @@ int fill_consts(ks_device *dev, const ks_scene *sc, const ks_camera_desc *cam, c
     rc.spp = p->spp;
     rc.seed = p->rng_seed;
     sobol_consts(rc.W, rc.H, rc.spp, rc.log2spp, rc.ndigits);
-    rc.perm_tab = dev->perm_tab.as<uint8_t>();
+    rc.perm_tab = dev->perm_tab.as<uint32_t>();
     KS_REQUIRE(2 * rc.ndigits <= 52 && (uint64_t)1 << rc.log2spp <= (uint64_t)rc.spp,
                "resolution x spp exceeds the sampler index range");
     rc.bounces = p->bounces;
@@ -2060,9 +2063,9 @@ int ks_device_open(int32_t ordinal, ks_device **out) {
         void *sp = nullptr;
         KS_HIP(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
         d->relmse_scratch = static_cast<double *>(sp);
-        KS_HIP(d->perm_tab.alloc((size_t)kPermTabDims * kPermTabPrefixes));
+        KS_HIP(d->perm_tab.alloc(sizeof(uint32_t) * (size_t)kPermTabDims * kPermTabPrefixes));
         hipLaunchKernelGGL(k_perm_tab, dim3(kPermTabDims * kPermTabPrefixes / 256), dim3(256), 0, d->stream,
-                           d->perm_tab.as<uint8_t>());
+                           d->perm_tab.as<uint32_t>());
         KS_HIP(hipGetLastError());
         KS_HIP(hipStreamSynchronize(d->stream));
         *out = d.release();
@@ -3505,7 +3508,7 @@ int ks_sobol_stream(ks_device *dev, int32_t width, int32_t height, int32_t spp, 
         KS_HIP(ou.alloc(sizeof(uint32_t) * n * n_values));
         KS_HIP(of.alloc(sizeof(float) * n * n_values));
         hipLaunchKernelGGL(k_sobol_stream, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n, dpx.p(), dpy.p(),
-                           ds.p(), seed, log2spp, ndigits, n_calls, dk.p(), n_values, dev->perm_tab.as<uint8_t>(),
+                           ds.p(), seed, log2spp, ndigits, n_calls, dk.p(), n_values, dev->perm_tab.as<uint32_t>(),
                            ou.as<uint32_t>(), of.as<float>());
         KS_HIP(hipGetLastError());
         KS_HIP(hipMemcpyAsync(out_u32, ou.p, sizeof(uint32_t) * n * n_values, hipMemcpyDeviceToHost, s));

@@ -115,29 +115,48 @@ KS_DEV uint32_t part_1_by_1(uint32_t x) {
     return x;
 }
 
-// The 24 base-4 digit permutations of sobol.h:171-197, one byte each (two bits per digit, in the
-// reference's order), packed four to a word and selected with compares instead of a memory access.
-KS_DEV uint32_t perm4_byte(uint32_t p) {
-    const uint32_t W0 = 0x78D8B4E4u, W1 = 0xB1E19C6Cu, W2 = 0x8D2D39C9u, W3 = 0x72D236C6u, W4 = 0x87271E4Eu,
-                   W5 = 0x93634B1Bu;
-    uint32_t w = p < 8 ? (p < 4 ? W0 : W1) : (p < 16 ? (p < 12 ? W2 : W3) : (p < 20 ? W4 : W5));
-    return (w >> ((p & 3u) * 8u)) & 0xffu;
-}
-// (mix_bits(x) >> 24) % 24 for a 32-bit x: the 40-bit quotient split at bit 32, with 2^32 = 16 mod 24.
-KS_DEV uint32_t perm_index(uint32_t x) {
-    uint64_t t = mix_bits((uint64_t)x) >> 24;
-    return ((uint32_t)(t >> 32) * 16u + (uint32_t)t % 24u) % 24u;
+// The 24 base-4 digit permutations of sobol.h:171-197, one byte each (two bits per digit), for index
+// (mix_bits(x) >> 24) % 24 of a 32-bit x. The index is never formed: an index mod 8 and mod 3 says which of
+// the 24 it is, so the bytes lie in three rows of eight (row = index mod 3, byte = index mod 8), picked by a
+// byte permute. mod 8 is three bits of the hash; mod 3, as 2^8 = 2^16 = 1, that of the sum of its bytes.
+// (With two 32-bit remainders by 24 and a select over six words the digit took about twenty more
+// instructions, four of them multiplies.)
+KS_DEV uint32_t perm4_of(uint32_t x) {
+    constexpr uint32_t kRow[3][2] = {{0x782739E4u, 0x72E14BC6u}, {0x872DB44Eu, 0xB163366Cu}, {0x8DD81EC9u, 0x93D29C1Bu}};
+    const uint64_t v = mix_bits((uint64_t)x);
+    const uint32_t hi = (uint32_t)(v >> 32), top = (uint32_t)v >> 24; // v >> 24 = hi 2^8 + top
+    uint32_t r = (hi & 0xffffu) + (hi >> 16) + top; // < 2^18, v >> 24 mod 3
+    r = (r & 0xffu) + (r >> 8);                     // <= 767
+    r -= 3u * ((r * 683u) >> 11);                   // exact up to 2046
+    const uint32_t k = top & 7u;
+    const uint32_t b0 = __builtin_amdgcn_perm(kRow[0][1], kRow[0][0], k);
+    const uint32_t b1 = __builtin_amdgcn_perm(kRow[1][1], kRow[1][0], k);
+    const uint32_t b2 = __builtin_amdgcn_perm(kRow[2][1], kRow[2][0], k);
+    return (r == 0u ? b0 : (r == 1u ? b1 : b2)) & 0xffu;
 }
 
-// Permutation bytes by (dimension, digit prefix): entry dim * kPermTabPrefixes + h is
-// perm4_byte(perm_index(h ^ 0x55555555 * dim)). A render's morton index is below 4^n_digits (2^(2 n_digits - 1)
-// for an odd log2 spp), so the prefix (the digits above) of each of the top kPermTabLevels digits has at
-// most 20 bits and is looked up; the lower digits' prefixes, and every digit of dimensions from
-// kPermTabDims on (paths of more than about 17 bounces), are hashed. The table is a constant of 128 MiB,
-// built once per device.
+// The permuted digits by (dimension, digit prefix): bits 0..19 of entry dim * kPermTabPrefixes + p are the ten
+// digits of p, each permuted by the digits above it, and bits 20..27 are the permutation byte of the digit
+// below p. A digit's permutation depends on the dimension and the digits above it alone, and leading zero
+// digits are digits like any other, so one table serves every render: the top ten digits of a sample index
+// and the eleventh cost one 4-byte load, where a byte table per digit took eleven loads and some 150
+// instructions of the 400 a sample took (k_shade is bound by its instructions). The lower digits, and
+// every digit of dimensions from kPermTabDims on (paths of more than about 17 bounces), are hashed. 512 MiB, a
+// constant, built once per device; a render reads the 4 MiB of each dimension it draws, mostly once
+// per pixel.
 constexpr uint32_t kPermTabDims = 128;
 constexpr uint32_t kPermTabPrefixes = 1u << 20;
-constexpr int kPermTabLevels = 11;
+constexpr int kPermTabDigits = 10;
+
+KS_DEV uint32_t perm_tab_entry(uint32_t dim, uint32_t p) {
+    const uint32_t dmask = 0x55555555u * dim;
+    uint32_t e = perm4_of(p ^ dmask) << (2 * kPermTabDigits);
+    for (int k = 0; k < kPermTabDigits; ++k) {
+        const uint32_t digit = (p >> (2 * k)) & 3u;
+        e |= ((perm4_of((p >> (2 * k + 2)) ^ dmask) >> (2 * digit)) & 3u) << (2 * k);
+    }
+    return e;
+}
 
 struct Sobol {
     uint32_t morton; // the reference's morton index is built from 32-bit parts (sobol.h:142-146)
@@ -145,11 +164,11 @@ struct Sobol {
     int32_t seed;
     int32_t log2_spp;
     int32_t n_digits;
-    const uint8_t *tab; // the permutation table above, or nullptr: every digit is hashed
+    const uint32_t *tab; // the table above, or nullptr: every digit is hashed
 
     // PTRenderSampler ctor: start_pixel with dimension 0 (sobol.h:142-146, 237-244)
     KS_DEV void start(uint32_t px, uint32_t py, uint32_t sample, int32_t dim0, int32_t seed_, int32_t log2spp,
-                      int32_t ndigits, const uint8_t *tab_ = nullptr) {
+                      int32_t ndigits, const uint32_t *tab_ = nullptr) {
         seed = seed_;
         log2_spp = log2spp;
         n_digits = ndigits;
@@ -158,57 +177,46 @@ struct Sobol {
         morton = (((part_1_by_1(py) << 1) + part_1_by_1(px)) << log2spp) | sample; // 32-bit as reference
     }
 
-    KS_DEV uint64_t sample_index() const { // sobol.h:168-222
-        uint64_t si = 0;
-        const bool pow2 = log2_spp & 1;
-        const int last = pow2 ? 1 : 0;
+    // The scrambled sample index (sobol.h:168-222), or its low 32 bits: T is uint64_t or uint32_t.
+    template <typename T> KS_DEV T sample_index() const {
+        const int odd = log2_spp & 1; // the lowest digit is a single bit
         const uint32_t dmask = 0x55555555u * (uint32_t)dim;
+        // digits above bit 31 of the 32-bit morton index are zero
+        auto from = [&](int shift) { return shift < 32 ? morton >> shift : 0u; };
+        auto put = [](uint32_t digits, int shift) {
+            return sizeof(T) == 8 || shift < 32 ? (T)((T)digits << shift) : (T)0;
+        };
+        T si = 0;
         int i = n_digits - 1;
-        if (tab != nullptr && (uint32_t)dim < kPermTabDims) {
-            // the top digits: their table loads are issued together, then applied
-            const uint8_t *t = tab + (size_t)dim * kPermTabPrefixes;
-            uint32_t pb[kPermTabLevels];
-#pragma unroll
-            for (int k = 0; k < kPermTabLevels; ++k) {
-                const int lv = n_digits - 1 - k;
-                const int shift = 2 * lv - (pow2 ? 1 : 0);
-                const uint32_t higher = lv >= last && shift + 2 < 32 ? morton >> (shift + 2) : 0u;
-                pb[k] = higher < kPermTabPrefixes ? t[higher] : perm4_byte(perm_index(higher ^ dmask));
+        const int low = n_digits - kPermTabDigits > odd ? n_digits - kPermTabDigits : odd; // lowest digit looked up
+        const uint32_t p = from(2 * low - odd);
+        if (tab != nullptr && (uint32_t)dim < kPermTabDims && p < kPermTabPrefixes) {
+            const uint32_t e = tab[(uint32_t)dim * kPermTabPrefixes + p];
+            si = put(e & ((1u << (2 * (n_digits - low))) - 1u), 2 * low - odd);
+            i = low - 1;
+            if (i >= odd) {
+                const int shift = 2 * i - odd;
+                si |= put((e >> (2 * kPermTabDigits + 2 * (from(shift) & 3u))) & 3u, shift);
+                --i;
             }
-#pragma unroll
-            for (int k = 0; k < kPermTabLevels; ++k) {
-                const int lv = n_digits - 1 - k;
-                if (lv < last) break;
-                const int shift = 2 * lv - (pow2 ? 1 : 0);
-                const uint32_t digit = shift < 32 ? (morton >> shift) & 3u : 0u;
-                si |= (uint64_t)((pb[k] >> (2 * digit)) & 3u) << shift;
-            }
-            i = n_digits - 1 - kPermTabLevels;
         }
-        for (; i >= last; --i) {
-            int shift = 2 * i - (pow2 ? 1 : 0);
-            // digits above bit 31 of the 32-bit morton index are zero
-            uint32_t digit = shift < 32 ? (morton >> shift) & 3u : 0u;
-            uint32_t higher = shift + 2 < 32 ? morton >> (shift + 2) : 0u;
-            uint32_t p = perm_index(higher ^ dmask);
-            digit = (perm4_byte(p) >> (2 * digit)) & 3u;
-            si |= (uint64_t)digit << shift;
+        for (; i >= odd; --i) {
+            const int shift = 2 * i - odd;
+            si |= put((perm4_of(from(shift + 2) ^ dmask) >> (2 * (from(shift) & 3u))) & 3u, shift);
         }
-        if (pow2) {
-            uint32_t digit = morton & 1u;
-            si |= (uint64_t)(digit ^ (uint32_t)(mix_bits((uint64_t)((morton >> 1) ^ dmask)) & 1u));
-        }
+        if (odd) si |= (T)((morton & 1u) ^ ((uint32_t)mix_bits((uint64_t)((morton >> 1) ^ dmask)) & 1u));
         return si;
     }
 
     KS_DEV uint32_t next_u32() { // sobol.h:148-155
-        uint64_t si = sample_index();
+        const uint32_t si = sample_index<uint32_t>(); // dimension 0 reads the low 32 bits alone
         ++dim;
         uint32_t h = (uint32_t)hash_dim_seed(dim, seed);
         return owen_scramble(sobol_dim0(si), h);
     }
     KS_DEV void next2d_u32(uint32_t &a, uint32_t &b) { // sobol.h:157-166
-        uint64_t si = sample_index();
+        // an index of at most 16 digits fits 32 bits (the same for every path of a render)
+        const uint64_t si = n_digits <= 16 ? sample_index<uint32_t>() : sample_index<uint64_t>();
         dim += 2;
         uint64_t bits = hash_dim_seed(dim, seed);
         a = owen_scramble(sobol_dim0(si), (uint32_t)bits);
