@@ -217,8 +217,7 @@ struct GridCorner {
     float w[8];
 };
 
-KS_DEV void grid_level_corners(const GuideNet &net, int level, const float u[3], GridCorner &c) {
-    uint32_t res = net.res[level];
+KS_DEV void grid_level_corners(uint32_t res, uint32_t level, uint32_t log2_T, const float u[3], GridCorner &c) {
     float res_f = (float)res;
     float p[3];
     uint32_t cell[3];
@@ -232,7 +231,7 @@ KS_DEV void grid_level_corners(const GuideNet &net, int level, const float u[3],
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
         uint32_t dx = k & 1, dy = (k >> 1) & 1, dz = (k >> 2) & 1;
-        c.idx[k] = grid_index(cell[0] + dx, cell[1] + dy, cell[2] + dz, res, net.log2_T) + ((uint32_t)level << net.log2_T);
+        c.idx[k] = grid_index(cell[0] + dx, cell[1] + dy, cell[2] + dz, res, log2_T) + (level << log2_T);
         c.w[k] = (dx ? p[0] : 1.0f - p[0]) * (dy ? p[1] : 1.0f - p[1]) * (dz ? p[2] : 1.0f - p[2]);
     }
 }
@@ -252,37 +251,6 @@ KS_DEV uint16_t f2bf(float f) {
 }
 KS_DEV float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 KS_DEV uint32_t bf_pair(float a, float b) { return (uint32_t)f2bf(a) | ((uint32_t)f2bf(b) << 16); }
-
-// Input row of one query, BF16: 32 grid features (level-major, FP32 trilinear sum of FP16 corners in
-// corner order 0..7), normal, wo, a constant 1 and zero padding to 64.
-KS_DEV void guide_encode(const GuideNet &net, f3 x, f3 n, f3 wo, uint16_t *row) {
-    float u[3];
-    normalise_position(net, x, u);
-    uint32_t *row32 = reinterpret_cast<uint32_t *>(row);
-    for (int l = 0; l < kGuideLevels; ++l) {
-        GridCorner c;
-        grid_level_corners(net, l, u, c);
-        float f0 = 0.0f, f1 = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            uint32_t v = net.grid_h[c.idx[k]];
-            f0 += c.w[k] * half_lo(v);
-            f1 += c.w[k] * half_hi(v);
-        }
-        row32[l] = bf_pair(f0, f1);
-    }
-    row32[16] = bf_pair(n.x, n.y);
-    row32[17] = bf_pair(n.z, wo.x);
-    row32[18] = bf_pair(wo.y, wo.z);
-    row32[19] = bf_pair(1.0f, 0.0f);
-#pragma unroll
-    for (int k = 20; k < kGuideIn / 2; ++k) row32[k] = 0u;
-}
-KS_DEV void guide_zero_row(uint16_t *row) {
-    uint32_t *row32 = reinterpret_cast<uint32_t *>(row);
-#pragma unroll
-    for (int k = 0; k < kGuideIn / 2; ++k) row32[k] = 0u;
-}
 
 // ---------------------------------------------------------------------------------------------------
 // BF16 and the MFMA tile helpers (v_mfma_f32_16x16x16_bf16; wave64)

@@ -200,7 +200,7 @@ __global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
 // Both features of one hash level: FP32 trilinear sum over corners 0..7.
 __device__ __forceinline__ void grid_pair(const GuideNet &net, int level, const float u[3], float &f0, float &f1) {
     GridCorner c;
-    grid_level_corners(net, level, u, c);
+    grid_level_corners(net.res[level], (uint32_t)level, net.log2_T, u, c);
     f0 = 0.0f;
     f1 = 0.0f;
 #pragma unroll
@@ -492,9 +492,15 @@ __global__ __launch_bounds__(256) void k_guide_fp8_pack(const float *mlp, const 
     }
 }
 
-// One wave per block. Every wave loops over chunks of 64 samples, accumulates the three weight
-// gradients in registers (MFMA) and scatters hash-grid gradients with FP32 atomics; at the end it writes
-// its weight-gradient partials (one slot per wave) for k_guide_reduce.
+// ---------------------------------------------------------------------------------------------------
+// Training: k_guide_encode -> k_guide_train -> k_guide_scatter (or k_guide_scatter_atomic), k_guide_reduce.
+// Samples are taken by position: position r of a slice of n holds sample (r % 64) * chunks + r / 64, chunks =
+// ceil(n / 64). Neighbours in the sample array come from neighbouring pixels and share their coarse grid
+// cells; 64 positions in a row lie far apart instead, so the lanes of a wave rarely add to one entry.
+// One kernel did all of it before, one wave per block at three waves per CU: 5.8 ms for 2^18 samples and a
+// 2^19-entry table, 4.3 ms with 2^16 entries. Encoding takes 0.09 ms at full occupancy, the layers 0.24 ms, the
+// scatter 0.61 (0.47) ms and the reduction 0.02 ms (0.18 before, one thread per parameter).
+// ---------------------------------------------------------------------------------------------------
 struct TrainSample {
     float4 xc; // position, weight c
     float4 n;
@@ -503,9 +509,56 @@ struct TrainSample {
 };
 static_assert(sizeof(TrainSample) == ksg::kTrainSampleBytes, "training sample layout");
 
-__global__ __launch_bounds__(64) void k_guide_train(GuideNet net, int n, int stride, const TrainSample *samples,
-                                                    float c_scale, float c_max, float *grid_grad, float *partials,
-                                                    double *loss_out, uint32_t *act_amax) {
+__device__ __forceinline__ uint32_t sample_at(uint32_t r, uint32_t chunks) { return (r & 63u) * chunks + (r >> 6); }
+
+// The network's input rows (64 BF16 each) and the normalised positions, by position; one thread per sample
+// and level, a wave holds four samples. Positions past the samples get zero rows.
+__global__ __launch_bounds__(256) void k_guide_encode(GuideNet net, uint32_t n, uint32_t stride, uint32_t chunks,
+                                                      const TrainSample *samples, uint32_t *rows, float4 *pos) {
+    __shared__ uint32_t s_res[kGuideLevels];
+    if (threadIdx.x < kGuideLevels) s_res[threadIdx.x] = net.res[threadIdx.x];
+    __syncthreads();
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    const uint32_t r = t / kGuideLevels, level = t % kGuideLevels;
+    if (r >= chunks * 64u) return;
+    const uint32_t i = sample_at(r, chunks);
+    uint32_t feature = 0u, rest = 0u;
+    if (i < n) {
+        const TrainSample *s = samples + (size_t)i * stride;
+        const float4 x = s->xc;
+        float u[3];
+        normalise_position(net, ld3(x), u);
+        GridCorner c;
+        grid_level_corners(s_res[level], level, net.log2_T, u, c);
+        float f0 = 0.0f, f1 = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t v = net.grid_h[c.idx[k]];
+            f0 += c.w[k] * half_lo(v);
+            f1 += c.w[k] * half_hi(v);
+        }
+        feature = bf_pair(f0, f1);
+        if (level < 4) { // normal, wo, a constant 1; the words after them stay zero
+            const float4 nn = s->n, wo = s->wo;
+            rest = level == 0 ? bf_pair(nn.x, nn.y) : level == 1 ? bf_pair(nn.z, wo.x) : level == 2 ? bf_pair(wo.y, wo.z)
+                                                                                                 : bf_pair(1.0f, 0.0f);
+        }
+        if (level == 0) pos[r] = make_float4(u[0], u[1], u[2], 0.0f);
+    } else if (level == 0) {
+        pos[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    rows[(size_t)r * (kGuideIn / 2) + level] = feature;
+    rows[(size_t)r * (kGuideIn / 2) + kGuideLevels + level] = rest;
+}
+
+// One wave per block. Every wave loops over chunks of 64 positions: forward, the head's and the layers'
+// backward, accumulating the three weight gradients in registers (MFMA). The gradient of the grid features
+// goes to dx, two floats per level and position, level after level. At the end the wave writes its
+// weight-gradient partials (one slot per wave) for k_guide_reduce.
+__global__ __launch_bounds__(64) void k_guide_train(GuideNet net, uint32_t n, uint32_t stride, uint32_t n_chunks,
+                                                    const TrainSample *samples, const uint32_t *rows, float c_scale,
+                                                    float c_max, float2 *dx, float *partials, double *loss_out,
+                                                    uint32_t *act_amax) {
     extern __shared__ __align__(16) uint8_t smem[];
     const int lane = threadIdx.x;
     const int r16 = lane & 15, q4 = (lane >> 4) * 4;
@@ -527,17 +580,24 @@ __global__ __launch_bounds__(64) void k_guide_train(GuideNet net, int n, int str
     }
     double loss = 0.0, wsum = 0.0, loss_cos = 0.0;
     float am[3] = {0.0f, 0.0f, 0.0f};
-    const int n_chunks = (n + 63) / 64;
-    for (int chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
-        int i = chunk * 64 + lane;
-        bool valid = i < n;
+    for (uint32_t chunk = blockIdx.x; chunk < n_chunks; chunk += gridDim.x) {
+        const uint32_t r = chunk * 64u + lane, i = sample_at(r, n_chunks);
+        const bool valid = i < n;
         TrainSample s{};
         if (valid) {
             s = samples[(size_t)i * stride];
             s.xc.w = fminf(s.xc.w * c_scale, c_max);
         }
-        if (valid) guide_encode(net, ld3(s.xc), ld3(s.n), ld3(s.wo), X + lane * kLdx);
-        else guide_zero_row(X + lane * kLdx);
+        { // the chunk's 64 rows of 128 B: eight lanes copy a row
+            const uint4 *src = reinterpret_cast<const uint4 *>(rows + (size_t)chunk * 64 * (kGuideIn / 2));
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const uint4 v = src[k * 64 + lane];
+                uint2 *dst = reinterpret_cast<uint2 *>(X + (k * 8 + lane / 8) * kLdx + (lane % 8) * 8);
+                dst[0] = make_uint2(v.x, v.y);
+                dst[1] = make_uint2(v.z, v.w);
+            }
+        }
         __syncthreads();
         wave_dense<4, true>(X, net.wt[0], H1, nullptr, 0);
         __syncthreads();
@@ -669,21 +729,11 @@ __global__ __launch_bounds__(64) void k_guide_train(GuideNet net, int n, int str
                 for (int r = 0; r < 4; ++r) DX[(m * 16 + q4 + r) * 32 + t * 16 + r16] = acc[t][r];
         }
         __syncthreads();
-        // hash-grid scatter
-        if (valid && s.xc.w > 0.0f) {
-            float u[3];
-            normalise_position(net, ld3(s.xc), u);
-            for (int l = 0; l < kGuideLevels; ++l) {
-                float d0 = DX[lane * 32 + 2 * l], d1 = DX[lane * 32 + 2 * l + 1];
-                if (d0 == 0.0f && d1 == 0.0f) continue;
-                GridCorner c;
-                grid_level_corners(net, l, u, c);
-                for (int k = 0; k < 8; ++k) {
-                    atomicAdd(&grid_grad[2 * (size_t)c.idx[k]], c.w[k] * d0);
-                    atomicAdd(&grid_grad[2 * (size_t)c.idx[k] + 1], c.w[k] * d1);
-                }
-            }
-        }
+        // the grid features' gradients, zero where the sample has no weight
+        const bool weighted = valid && s.xc.w > 0.0f;
+        for (int l = 0; l < kGuideLevels; ++l)
+            dx[(size_t)l * n_chunks * 64u + r] = weighted ? make_float2(DX[lane * 32 + 2 * l], DX[lane * 32 + 2 * l + 1])
+                                                          : make_float2(0.0f, 0.0f);
         __syncthreads();
     }
     // weight-gradient partials of this wave in [in][out] order
@@ -716,12 +766,103 @@ __global__ __launch_bounds__(64) void k_guide_train(GuideNet net, int n, int str
     }
 }
 
-__global__ void k_guide_reduce(const float *partials, int n_waves, float *grad_mlp) {
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= kMlpParams) return;
+// The grid's gradient, added up in LDS: a block owns kScatterEntries entries of one level and goes over the
+// positions of its share, keeping what falls in its entries (tiles: level, first entry, entries, share | shares
+// << 16). Global float atomics take 47 ps each on this card wherever they fall (67 M of a 2^18-sample step: 3.2
+// ms, 5 ms where lanes share entries), nearly the whole of the step; here a position costs a tile about a
+// hundred instructions and its hits LDS atomics. Levels of few tiles are shared out over the positions so
+// that every block has about as many hits. The only share of a tile writes its entries (adds them with
+// `add`: earlier slices' sums), the others add what is not zero to cleared memory.
+constexpr uint32_t kScatterEntries = 16384; // 128 KB of float pairs
+constexpr uint32_t kScatterShares = 16;      // blocks a hashed level is given at least
+constexpr uint32_t kScatterDenseShares = 64; // and a dense one, whose surfaces fill few of its tiles
+constexpr int kScatterBlock = 1024;
+__global__ __launch_bounds__(kScatterBlock) void k_guide_scatter(GuideNet net, uint32_t positions, const float4 *pos,
+                                                                 const float2 *dx, const uint4 *tiles, float *grid_grad,
+                                                                 int add) {
+    __shared__ float s_sum[2][kScatterEntries]; // a plane per feature: hits spread over all banks
+    const uint4 tile = tiles[blockIdx.x];
+    const uint32_t level = tile.x, first = tile.y, count = tile.z, share = tile.w & 0xffffu, shares = tile.w >> 16;
+    const uint32_t res = net.res[level];
+    for (uint32_t e = threadIdx.x; e < count; e += kScatterBlock) s_sum[0][e] = s_sum[1][e] = 0.0f;
+    __syncthreads();
+    const float2 *d = dx + (size_t)level * positions;
+    const uint32_t base = first + (level << net.log2_T); // corner indices carry their level
+    const uint32_t step = shares * kScatterBlock, start = share * kScatterBlock + threadIdx.x;
+    float4 p_next = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float2 d_next = make_float2(0.0f, 0.0f);
+    if (start < positions) {
+        p_next = pos[start];
+        d_next = d[start];
+    }
+    for (uint32_t r = start; r < positions; r += step) {
+        const float4 p = p_next;
+        const float2 g = d_next;
+        if (r + step < positions) { // the next position's loads run under this one's work
+            p_next = pos[r + step];
+            d_next = d[r + step];
+        }
+        if (g.x == 0.0f && g.y == 0.0f) continue;
+        const float u[3] = {p.x, p.y, p.z};
+        GridCorner c;
+        grid_level_corners(res, level, net.log2_T, u, c);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const uint32_t e = c.idx[k] - base;
+            if (e < count) {
+                atomicAdd(&s_sum[0][e], c.w[k] * g.x);
+                atomicAdd(&s_sum[1][e], c.w[k] * g.y);
+            }
+        }
+    }
+    __syncthreads();
+    float2 *out = reinterpret_cast<float2 *>(grid_grad) + base;
+    for (uint32_t e = threadIdx.x; e < count; e += kScatterBlock) {
+        const float a = s_sum[0][e], b = s_sum[1][e];
+        if (shares == 1) {
+            const float2 o = add ? out[e] : make_float2(0.0f, 0.0f);
+            out[e] = make_float2(o.x + a, o.y + b);
+        } else if (a != 0.0f || b != 0.0f) {
+            atomicAdd(&out[e].x, a);
+            atomicAdd(&out[e].y, b);
+        }
+    }
+}
+
+// The same with global atomics, one thread per level and position, for tables of so many tiles that going
+// over all positions for each costs more.
+__global__ __launch_bounds__(256) void k_guide_scatter_atomic(GuideNet net, uint32_t positions, const float4 *pos,
+                                                              const float2 *dx, float *grid_grad) {
+    const uint32_t level = blockIdx.y, r = blockIdx.x * 256u + threadIdx.x;
+    if (r >= positions) return;
+    const float2 g = dx[(size_t)level * positions + r];
+    if (g.x == 0.0f && g.y == 0.0f) return;
+    const float4 p = pos[r];
+    const float u[3] = {p.x, p.y, p.z};
+    GridCorner c;
+    grid_level_corners(net.res[level], level, net.log2_T, u, c);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        atomicAdd(&grid_grad[2 * (size_t)c.idx[k]], c.w[k] * g.x);
+        atomicAdd(&grid_grad[2 * (size_t)c.idx[k] + 1], c.w[k] * g.y);
+    }
+}
+
+// Weight gradients: the waves' partials summed in wave order by 16 threads per parameter (each every 16th
+// wave), then over the 16.
+__global__ __launch_bounds__(256) void k_guide_reduce(const float *partials, int n_waves, float *grad_mlp, int add) {
+    __shared__ float s_sum[16][16];
+    const int p = blockIdx.x * 16 + (threadIdx.x & 15), part = threadIdx.x >> 4;
     float s = 0.0f;
-    for (int w = 0; w < n_waves; ++w) s += partials[(size_t)w * kMlpParams + p];
-    grad_mlp[p] = s;
+    if (p < kMlpParams)
+        for (int w = part; w < n_waves; w += 16) s += partials[(size_t)w * kMlpParams + p];
+    s_sum[part][threadIdx.x & 15] = s;
+    __syncthreads();
+    if (part == 0 && p < kMlpParams) {
+        float t = 0.0f;
+        for (int k = 0; k < 16; ++k) t += s_sum[k][threadIdx.x];
+        grad_mlp[p] = add ? grad_mlp[p] + t : t;
+    }
 }
 
 // Adam (gpu/shaders/adam.slang:39-50) over every parameter; refreshes the low-precision copies and
@@ -917,6 +1058,9 @@ struct ks_guide {
     uint32_t res[kGuideLevels];
     float lo[3], inv_ext[3];
     DevBuf params, grad, m1, m2, grid_h, w_bf, wt_bf, partials, loss, samples;
+    DevBuf rows, pos, dx; // a training slice's input rows, normalised positions and feature gradients
+    DevBuf tiles;         // k_guide_scatter's tiles (n_tiles; 0: the table is scattered with atomics)
+    uint32_t n_tiles = 0;
     DevBuf w8, fp8s, act_amax; // FP8 copy of the MLP, its scales, recorded activation maxima
     bool fp8 = false;          // inference in FP8
     int32_t n_partials = 0;
@@ -993,24 +1137,52 @@ int launch_extract(const float4 *recs, const float4 *samp, uint32_t n_items, uin
     return KS_OK;
 }
 
+// Loss, weight gradients and grid gradient of n device-resident samples (TrainSample records, every
+// stride-th one) into g->loss and g->grad, whose grid part must be zero (as Adam leaves it). Slices of at most kTrainSlice samples bound the
+// buffers (288 B a sample).
+constexpr int64_t kTrainSlice = 1 << 20;
+int gradient_on_device(ks_guide *g, const TrainSample *samples, int64_t n, int stride, float c_scale, float c_max,
+                       uint32_t *act_amax, hipStream_t s) {
+    const GuideNet net = net_of(g);
+    KS_HIP(hipMemsetAsync(g->loss.p, 0, 3 * sizeof(double), s));
+    for (int64_t first = 0; first < n; first += kTrainSlice) {
+        const uint32_t m = (uint32_t)std::min<int64_t>(kTrainSlice, n - first), chunks = (m + 63u) / 64u;
+        const uint32_t positions = chunks * 64u;
+        const TrainSample *slice = samples + first * stride;
+        const int add = first > 0 ? 1 : 0;
+        const int waves = (int)std::min<uint32_t>(chunks, (uint32_t)std::max(1, ksg::device_cu_count(g->dev) * 3));
+        KS_HIP(g->partials.ensure(sizeof(float) * (size_t)waves * kMlpParams));
+        KS_HIP(g->rows.ensure(sizeof(uint32_t) * (kGuideIn / 2) * (size_t)positions));
+        KS_HIP(g->pos.ensure(sizeof(float4) * (size_t)positions));
+        KS_HIP(g->dx.ensure(sizeof(float2) * kGuideLevels * (size_t)positions));
+        hipLaunchKernelGGL(k_guide_encode, dim3(positions * kGuideLevels / 256u), dim3(256), 0, s, net, m, (uint32_t)stride,
+                           chunks, slice, g->rows.as<uint32_t>(), g->pos.as<float4>());
+        hipLaunchKernelGGL(k_guide_train, dim3(waves), dim3(64), kTrainWaveBytes, s, net, m, (uint32_t)stride, chunks,
+                           slice, g->rows.as<uint32_t>(), c_scale, c_max, g->dx.as<float2>(), g->partials.as<float>(),
+                           g->loss.as<double>(), act_amax);
+        if (g->n_tiles > 0)
+            hipLaunchKernelGGL(k_guide_scatter, dim3(g->n_tiles), dim3(kScatterBlock), 0, s, net, positions,
+                               g->pos.as<float4>(), g->dx.as<float2>(), g->tiles.as<uint4>(), g->grad.as<float>(), add);
+        else
+            hipLaunchKernelGGL(k_guide_scatter_atomic, dim3((positions + 255u) / 256u, kGuideLevels), dim3(256), 0, s, net,
+                               positions, g->pos.as<float4>(), g->dx.as<float2>(), g->grad.as<float>());
+        hipLaunchKernelGGL(k_guide_reduce, dim3((kMlpParams + 15) / 16), dim3(256), 0, s, g->partials.as<float>(), waves,
+                           g->grad.as<float>() + g->n_grid, add);
+        KS_HIP(hipGetLastError());
+    }
+    return KS_OK;
+}
+
 // One Adam step on n device-resident samples (TrainSample records, every stride-th one).
 int train_on_device(ks_guide *g, const void *samples, int n, int stride, float c_scale, double *loss_host,
                     hipStream_t s) {
     if (n <= 0) return KS_OK;
-    int n_chunks = (n + 63) / 64;
-    int waves = std::min(n_chunks, std::max(1, ksg::device_cu_count(g->dev) * 3));
-    KS_HIP(g->partials.ensure(sizeof(float) * (size_t)waves * kMlpParams));
-    KS_HIP(hipMemsetAsync(g->loss.p, 0, 3 * sizeof(double), s));
     // with FP8 inference the step's forward records the activation maxima that scale the next FP8 copy
     if (g->fp8) KS_HIP(hipMemsetAsync(g->act_amax.p, 0, 3 * sizeof(uint32_t), s));
     const float c_max = c_scale > 0.0f && g->cfg.weight_clamp > 0.0f ? g->cfg.weight_clamp : INFINITY;
-    hipLaunchKernelGGL(k_guide_train, dim3(waves), dim3(64), kTrainWaveBytes, s, net_of(g), n, stride,
-                       static_cast<const TrainSample *>(samples), c_scale > 0.0f ? c_scale : 1.0f, c_max,
-                       g->grad.as<float>(), g->partials.as<float>(), g->loss.as<double>(),
-                       g->fp8 ? g->act_amax.as<uint32_t>() : nullptr);
-    KS_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_guide_reduce, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, g->partials.as<float>(), waves,
-                       g->grad.as<float>() + g->n_grid);
+    int ge = gradient_on_device(g, static_cast<const TrainSample *>(samples), n, stride, c_scale > 0.0f ? c_scale : 1.0f,
+                                c_max, g->fp8 ? g->act_amax.as<uint32_t>() : nullptr, s);
+    if (ge) return ge;
     g->steps += 1;
     g->samples_used += n;
     float bc1 = 1.0f - std::pow(g->cfg.beta1, (float)g->steps), bc2 = 1.0f - std::pow(g->cfg.beta2, (float)g->steps);
@@ -1087,6 +1259,30 @@ int ks_guide_create(ks_device *dev, const ks_guide_config *cfg_in, const float b
         KS_HIP(g->w_bf.alloc(sizeof(uint16_t) * kMlpParams));
         KS_HIP(g->wt_bf.alloc(sizeof(uint16_t) * kMlpParams));
         KS_HIP(g->loss.alloc(3 * sizeof(double)));
+        {
+            // k_guide_scatter's tiles: the entries a level uses (all of a dense level's, else the table), in runs
+            // of kScatterEntries. Entries past a dense level's are never touched; their gradient stays zero.
+            std::vector<uint4> tiles;
+            for (int l = 0; l < kGuideLevels; ++l) {
+                const uint64_t side = (uint64_t)g->res[l] + 1, dense = side * side * side, T = 1ull << g->log2_T;
+                const uint32_t used = (uint32_t)std::min(dense, T);
+                const uint32_t n = (used + kScatterEntries - 1) / kScatterEntries;
+                const uint32_t shares = std::max(1u, (dense <= T ? kScatterDenseShares : kScatterShares) / n);
+                for (uint32_t e = 0; e < used; e += kScatterEntries)
+                    for (uint32_t k = 0; k < shares; ++k)
+                        tiles.push_back(
+                            make_uint4((uint32_t)l, e, std::min(kScatterEntries, used - e), k | (shares << 16)));
+            }
+            // A position costs a round of 256 tiles about 0.65 ns and 256 atomics 12 ns: atomics from 16 rounds on
+            // (tables of 2^22 entries and more).
+            if (tiles.size() < 4096) {
+                g->n_tiles = (uint32_t)tiles.size();
+                KS_HIP(g->tiles.alloc(sizeof(uint4) * tiles.size()));
+                KS_HIP(hipMemcpyAsync(g->tiles.p, tiles.data(), sizeof(uint4) * tiles.size(), hipMemcpyHostToDevice,
+                                      g->stream));
+                KS_HIP(hipStreamSynchronize(g->stream));
+            }
+        }
         KS_HIP(g->w8.alloc(sizeof(uint64_t) * kFp8Frags));
         KS_HIP(g->fp8s.alloc(sizeof(float) * kFp8ScaleCount));
         KS_HIP(g->act_amax.alloc(sizeof(uint32_t) * 3));
@@ -1259,18 +1455,9 @@ int ks_guide_gradient(ks_guide *g, int64_t n, const float *queries, const float 
         int e = upload_samples(g, n, queries, wi, weight);
         if (e) return e;
         hipStream_t s = g->stream;
-        int n_chunks = (int)((n + 63) / 64);
-        int waves = std::min(n_chunks, std::max(1, ksg::device_cu_count(g->dev) * 3));
-        KS_HIP(g->partials.ensure(sizeof(float) * (size_t)waves * kMlpParams));
-        KS_HIP(hipMemsetAsync(g->loss.p, 0, 3 * sizeof(double), s));
         KS_HIP(hipMemsetAsync(g->grad.p, 0, sizeof(float) * g->n_grid, s));
-        hipLaunchKernelGGL(k_guide_train, dim3(waves), dim3(64), kTrainWaveBytes, s, ksg::net_of(g), (int)n, 1,
-                           g->samples.as<TrainSample>(), 1.0f, INFINITY, g->grad.as<float>(), g->partials.as<float>(),
-                           g->loss.as<double>(), nullptr);
-        KS_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_guide_reduce, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, g->partials.as<float>(), waves,
-                           g->grad.as<float>() + g->n_grid);
-        KS_HIP(hipGetLastError());
+        e = ksg::gradient_on_device(g, g->samples.as<TrainSample>(), n, 1, 1.0f, INFINITY, nullptr, s);
+        if (e) return e;
         KS_HIP(hipMemcpyAsync(grad, g->grad.p, sizeof(float) * (g->n_grid + kMlpParams), hipMemcpyDeviceToHost, s));
         if (loss) KS_HIP(hipMemcpyAsync(loss, g->loss.p, sizeof(double), hipMemcpyDeviceToHost, s));
         KS_HIP(hipMemsetAsync(g->grad.p, 0, sizeof(float) * (g->n_grid + kMlpParams), s));

@@ -1,0 +1,73 @@
+"""The grid gradient's accumulation at its edges: batches of one sample, of a wave, of a scatter block and one
+more or less, a batch of more than one slice, and a table whose tiles are so many that it is scattered
+with global atomics. Against the oracle's gradient of the same BF16 operands (bar of test_gpu_guide.py), the
+slices against the sum of their parts."""
+
+import numpy as np
+import pytest
+
+import ks_guide_oracle as go
+from test_gpu_guide import BOUNDS, CONFIGS, _params, _queries
+
+pytestmark = pytest.mark.gpu
+
+
+def _samples(rng, n):
+    q = _queries(rng, n, BOUNDS[0], BOUNDS[1])
+    wi = rng.standard_normal((n, 3)).astype(np.float32)
+    return q, wi, rng.uniform(0.05, 2.0, n).astype(np.float32)
+
+
+def _check(g, lay, n, seed):
+    rng = np.random.default_rng(seed)
+    p = _params(g.n_grid, rng)
+    g.set_params(p)
+    s = _samples(rng, n)
+    loss, grad = g.gradient(*s)
+    l_ref, g_ref = go.gradient(p, lay, *s, quantised=True)
+    assert loss == pytest.approx(l_ref, rel=1e-4)
+    o = g.n_grid
+    for a, b in ((0, o), (o, o + go.MLP_SIZE)):
+        assert np.linalg.norm(grad[a:b] - g_ref[a:b]) < 5e-3 * np.linalg.norm(g_ref[a:b])
+    assert np.array_equal(grad[:o] != 0, g_ref[:o] != 0)
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025])
+@pytest.mark.parametrize("log2_T", [12, 15])  # tiles of one and of several per level, shared over positions
+def test_batch_edges(ks, device, n, log2_T):
+    print("scatter", n, log2_T, flush=True)
+    cfg = dict(CONFIGS["small"], log2_table_size=log2_T)
+    g = ks.Guide(device, *BOUNDS, ks.guide_config(seed=7, **cfg))
+    _check(g, go.Layout(log2_T, 4.0, 256.0, *BOUNDS), n, n)
+    g.close()
+
+
+def test_large_table_uses_atomics(ks, device):
+    """Sixteen hashed levels of 2^22 entries: 4096 tiles."""
+    print("scatter atomics", flush=True)
+    g = ks.Guide(device, *BOUNDS, ks.guide_config(seed=7, log2_table_size=22, base_resolution=256.0, max_resolution=512.0))
+    _check(g, go.Layout(22, 256.0, 512.0, *BOUNDS), 130, 5)
+    g.close()
+
+
+def test_slices_add_up(ks, device):
+    """2^20 + 130 samples are two slices. Each entry's sum of m FP32 terms errs by at most m 2^-24 of the terms'
+    absolute sum, about sqrt(m) 2^-24 when rounding errors are independent: below 1e-4 for the 2^20 terms that
+    meet in a weight, with an allowance of 4 for cancellation between them."""
+    print("scatter slices", flush=True)
+    g = ks.Guide(device, *BOUNDS, ks.guide_config(seed=7, **CONFIGS["small"]))
+    rng = np.random.default_rng(9)
+    g.set_params(_params(g.n_grid, rng))
+    q, wi, c = _samples(rng, (1 << 20) + 130)
+    k = 1 << 20
+    l0, g0 = g.gradient(q[:k], wi[:k], c[:k])
+    l1, g1 = g.gradient(q[k:], wi[k:], c[k:])
+    loss, grad = g.gradient(q, wi, c)
+    assert loss == pytest.approx(l0 + l1, rel=1e-9)
+    o = g.n_grid
+    for a, b in ((0, o), (o, o + go.MLP_SIZE)):
+        want = g0[a:b].astype(np.float64) + g1[a:b]
+        err = np.linalg.norm(grad[a:b] - want) / np.linalg.norm(want)
+        print("relative L2 difference", err, flush=True)
+        assert err < 4e-4
+    g.close()
