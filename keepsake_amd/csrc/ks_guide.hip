@@ -185,14 +185,26 @@ struct QueryList {
     }
 };
 
+// One counter takes one block's atomic every 11.5 ns, so a block appends the queries of kCompactPer x 256
+// paths with one (with one per 256 paths the 7.4 M of a 720p 8-spp pass took 332 us, nearly all of it the
+// 28800 atomics).
+constexpr int kCompactPer = 8;
 __global__ __launch_bounds__(256) void k_guide_compact(QueryHits h, Queue q, uint32_t *list, uint32_t *n_list) {
-    __shared__ uint32_t s_app[5];
+    __shared__ uint32_t s_slot[kCompactPer * 4 + 1];
     const uint32_t n = q.active();
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (blockIdx.x * blockDim.x >= n) return;
-    const bool want = i < n && h.wanted(i);
-    const uint32_t j = block_append<4>(n_list, want, s_app);
-    if (want) list[j] = i;
+    const uint32_t first = blockIdx.x * (256u * kCompactPer);
+    if (first >= n) return;
+    uint64_t mask[kCompactPer];
+#pragma unroll
+    for (int k = 0; k < kCompactPer; ++k) {
+        const uint32_t i = first + k * 256u + threadIdx.x;
+        mask[k] = __ballot(i < n && h.wanted(i));
+    }
+    const uint32_t base = block_slots<kCompactPer>(mask, n_list, s_slot);
+#pragma unroll
+    for (int k = 0; k < kCompactPer; ++k)
+        if ((mask[k] >> __lane_id()) & 1ull)
+            list[base + s_slot[k * 4 + (threadIdx.x >> 6)] + lanes_below(mask[k])] = first + k * 256u + threadIdx.x;
 }
 
 __global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
@@ -982,41 +994,56 @@ __global__ void k_vmm_sample(int64_t n, const float *mix, const float *u, float 
     pdf[i] = mixture_pdf(m, w);
 }
 
-// One thread per record slot: work item w = slot / kRecVertices. The final sample value of a pass with
-// one sample per pixel sits at samp[w].
-__global__ void k_guide_extract(const float4 *recs, const float4 *samp, uint32_t n_items, uint32_t stamp,
-                                TrainSample *out, uint32_t *count, double *c_sum, uint32_t cap) {
-    const uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-    bool take = false;
-    TrainSample t{};
-    if (slot < n_items * (uint32_t)kRecVertices) {
-        const float4 *r = recs + (size_t)slot * kRecFloat4;
-        float4 x = r[0];
-        if (__float_as_uint(x.w) == stamp) {
-            f3 Lf = ld3(samp[slot / kRecVertices]);
-            f3 d = Lf - ld3(r[4]) - ld3(r[kRecNee]);
-            f3 b = ld3(r[5]);
-            f3 X = mk(b.x > 0.0f ? d.x / b.x : 0.0f, b.y > 0.0f ? d.y / b.y : 0.0f, b.z > 0.0f ? d.z / b.z : 0.0f);
-            float c = luminance(X);
-            if (c > 0.0f && isfinite(c)) {
-                take = true;
-                t.xc = make_float4(x.x, x.y, x.z, c);
-                t.n = r[1];
-                t.wo = r[2];
-                t.wi = r[3];
+// kExtractPer record slots per thread: work item w = slot / kRecVertices. The final sample value of a pass with
+// one sample per pixel sits at samp[w]. One atomic per block on each of the two totals: with one per wave
+// the 2.8 M slots of a 720p pass took 965 us, the time of 2 x 43200 atomics on two addresses.
+constexpr int kExtractPer = 8;
+__global__ __launch_bounds__(256) void k_guide_extract(const float4 *recs, const float4 *samp, uint32_t n_items,
+                                                       uint32_t stamp, TrainSample *out, uint32_t *count, double *c_sum,
+                                                       uint32_t cap) {
+    __shared__ uint32_t s_slot[kExtractPer * 4 + 1];
+    __shared__ double s_sum[4];
+    const uint32_t first = blockIdx.x * (256u * kExtractPer) + threadIdx.x, n = n_items * (uint32_t)kRecVertices;
+    float weight[kExtractPer];
+    uint64_t mask[kExtractPer];
+    double cs = 0.0;
+#pragma unroll
+    for (int k = 0; k < kExtractPer; ++k) {
+        const uint32_t slot = first + k * 256u;
+        float c = 0.0f;
+        if (slot < n) {
+            const float4 *r = recs + (size_t)slot * kRecFloat4;
+            if (__float_as_uint(r[0].w) == stamp) {
+                f3 d = ld3(samp[slot / kRecVertices]) - ld3(r[4]) - ld3(r[kRecNee]);
+                f3 b = ld3(r[5]);
+                f3 X = mk(b.x > 0.0f ? d.x / b.x : 0.0f, b.y > 0.0f ? d.y / b.y : 0.0f, b.z > 0.0f ? d.z / b.z : 0.0f);
+                c = luminance(X);
+                if (!(c > 0.0f && isfinite(c))) c = 0.0f;
             }
         }
+        weight[k] = c;
+        mask[k] = __ballot(c > 0.0f);
+        cs += (double)c;
     }
-    double cs = take ? (double)t.xc.w : 0.0;
     for (int off = 32; off > 0; off >>= 1) cs += __shfl_xor(cs, off);
-    if (__lane_id() == 0 && cs != 0.0) atomicAdd(c_sum, cs);
-    uint32_t j = wave_append(count, take);
-    if (take && j < cap) {
+    if (__lane_id() == 0) s_sum[threadIdx.x >> 6] = cs;
+    const uint32_t base = block_slots<kExtractPer>(mask, count, s_slot); // synchronises the block
+    if (threadIdx.x == 0) {
+        const double t = s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3];
+        if (t != 0.0) atomicAdd(c_sum, t);
+    }
+#pragma unroll
+    for (int k = 0; k < kExtractPer; ++k) {
+        if (!((mask[k] >> __lane_id()) & 1ull)) continue;
+        const uint32_t j = base + s_slot[k * 4 + (threadIdx.x >> 6)] + lanes_below(mask[k]);
+        if (j >= cap) continue;
+        const float4 *r = recs + (size_t)(first + k * 256u) * kRecFloat4;
+        const float4 x = r[0];
         TrainSample *o = out + j;
-        o->xc = t.xc;
-        o->n = t.n;
-        o->wo = t.wo;
-        o->wi = t.wi;
+        o->xc = make_float4(x.x, x.y, x.z, weight[k]);
+        o->n = r[1];
+        o->wo = r[2];
+        o->wi = r[3];
     }
 }
 
@@ -1105,7 +1132,8 @@ int launch_infer(ks_guide *g, const DevScene &sc, const Queue &q, uint32_t block
                  uint32_t *n_list, hipStream_t s) {
     const QueryHits qh{sc, rd, hits, state, max_bounce};
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, n_list);
-    hipLaunchKernelGGL(k_guide_compact, dim3(blocks), dim3(256), 0, s, qh, q, list, n_list);
+    hipLaunchKernelGGL(k_guide_compact, dim3((blocks + kCompactPer - 1) / kCompactPer), dim3(256), 0, s, qh, q, list,
+                       n_list);
     static_assert(kInferBlock == 256, "the inference launch covers as many queries as the shading launch");
     const QueryList ql{qh, list, n_list};
     if (g->fp8)
@@ -1131,7 +1159,8 @@ int64_t guide_steps(const ks_guide *g) { return g->steps; }
 int launch_extract(const float4 *recs, const float4 *samp, uint32_t n_items, uint32_t stamp, void *out,
                    uint32_t *count, double *c_sum, uint32_t cap, hipStream_t s) {
     uint64_t slots = (uint64_t)n_items * kRecVertices;
-    hipLaunchKernelGGL(k_guide_extract, dim3((unsigned)((slots + 255) / 256)), dim3(256), 0, s, recs, samp, n_items,
+    hipLaunchKernelGGL(k_guide_extract, dim3((unsigned)((slots + 256 * kExtractPer - 1) / (256 * kExtractPer))), dim3(256),
+                       0, s, recs, samp, n_items,
                        stamp, static_cast<TrainSample *>(out), count, c_sum, cap);
     KS_HIP(hipGetLastError());
     return KS_OK;

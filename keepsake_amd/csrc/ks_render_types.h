@@ -138,19 +138,6 @@ struct GuideShade {
 // ---------------------------------------------------------------------------------------------------
 // Wave-level helpers (wave64)
 // ---------------------------------------------------------------------------------------------------
-KS_DEV uint32_t wave_append(uint32_t *counter, bool pred) {
-    uint64_t mask = __ballot(pred);
-    uint32_t lane = __lane_id();
-    uint32_t prefix = __popcll(mask & ((1ull << lane) - 1ull));
-    uint32_t base = 0;
-    if (mask != 0) {
-        int leader = __ffsll((unsigned long long)mask) - 1;
-        if ((int)lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-        base = __shfl(base, leader);
-    }
-    return base + prefix;
-}
-
 // Block-level append: the block's slots come from one atomic per block rather than one per wave (many
 // blocks appending to one counter serialise on its atomic unit). Every thread of the block must call it,
 // as it synchronises the block; s_tmp is NWAVES + 1 words of LDS. Slots follow wave order, then lane
@@ -202,6 +189,29 @@ KS_DEV void block_append2(uint32_t *counter_a, bool a, uint32_t *counter_b, bool
     __syncthreads();
     slot_a = s_tmp[NWAVES] + s_tmp[wave] + (uint32_t)__popcll(mask_a & below);
     slot_b = s_tmp[2 * NWAVES + 1] + s_tmp[NWAVES + 1 + wave] + (uint32_t)__popcll(mask_b & below);
+}
+
+// This lane's place among the lanes of a ballot mask.
+KS_DEV uint32_t lanes_below(uint64_t mask) { return (uint32_t)__popcll(mask & ((1ull << __lane_id()) - 1ull)); }
+
+// Slots for PER ballots of each of a block's four waves, with one atomic on the counter: returns the block's
+// first slot and leaves in s_slot[k * 4 + wave] the offset of ballot k of a wave (s_slot: PER * 4 + 1 words
+// of LDS). Every thread of the block calls it; it synchronises the block.
+template <int PER> KS_DEV uint32_t block_slots(const uint64_t (&mask)[PER], uint32_t *counter, uint32_t *s_slot) {
+    if (__lane_id() == 0)
+        for (int k = 0; k < PER; ++k) s_slot[k * 4 + (threadIdx.x >> 6)] = (uint32_t)__popcll(mask[k]);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t total = 0;
+        for (int e = 0; e < PER * 4; ++e) {
+            const uint32_t c = s_slot[e];
+            s_slot[e] = total;
+            total += c;
+        }
+        s_slot[PER * 4] = total ? atomicAdd(counter, total) : 0u;
+    }
+    __syncthreads();
+    return s_slot[PER * 4];
 }
 
 // Adds per-lane counts into this block's own row of `rows` (kStatCount slots per row): wave sums by
