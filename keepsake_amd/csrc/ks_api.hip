@@ -287,11 +287,12 @@ template <bool BATCH> __global__ __launch_bounds__(256) void k_raygen(RenderCons
 
 // Closest hit for n rays (count read from *n_dev when given). Grid-stride over rays; one LDS stack
 // column per lane. Ray, node and triangle counts go to the block's row of stat_rows.
-// The traversal kernels run at 8 waves per SIMD (64 VGPRs). With ALPHA they call the opacity test, and a
-// call within 64 VGPRs spilled the traversal loop's state to scratch on every node visit; they are held
-// to 4 waves per SIMD (128 VGPRs) instead, with no spills.
+// The traversal kernels run at 8 waves per SIMD (64 VGPRs), the alpha-tested ones, with the opacity test inlined,
+// at 5: textured 509 x 383, 16 spp, traversal per render 7.84 ms at 4 waves (108 VGPRs), 7.54 at 5, 7.96 at 6; as
+// a call the test took 448 B of scratch a lane and 9.68 ms (4 waves).
+constexpr int kAlphaTraceWaves = 5;
 template <int W, bool ALPHA>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? 4 : 8))) void k_closest(DevScene sc, const uint32_t *n_dev, uint32_t n_fixed,
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? kAlphaTraceWaves : 8))) void k_closest(DevScene sc, const uint32_t *n_dev, uint32_t n_fixed,
                                                          const float4 *ro, const float4 *rd, float4 *hit,
                                                          uint32_t *ovf, uint32_t ovf_cap,
                                                          unsigned long long *stat_rows) {
@@ -345,7 +346,7 @@ KS_DEV void add_nee(uint32_t i, const uint32_t *target, const float4 *contrib, f
 
 // Any hit: the occlusion flag of each of n rays (ks_occluded).
 template <int W, bool ALPHA>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? 4 : 8))) void k_anyhit(DevScene sc, const uint32_t *n_dev, uint32_t n_fixed,
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? kAlphaTraceWaves : 8))) void k_anyhit(DevScene sc, const uint32_t *n_dev, uint32_t n_fixed,
                                                         const float4 *ro, const float4 *rd, uint8_t *occ,
                                                         uint32_t *ovf, uint32_t ovf_cap,
                                                         unsigned long long *stat_rows) {
@@ -385,7 +386,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALP
 // LDS totals of the ray's kind when it ends (no per-kind registers in the loop). Block 0 adds the ray counts
 // and prepares the counters that the iteration's shading pass appends to.
 template <int W, bool ALPHA>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? 4 : 8))) void k_trace(
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(ALPHA ? kAlphaTraceWaves : 8))) void k_trace(
     DevScene sc, Queue q, uint32_t closest, const float4 *ro, const float4 *rd, float4 *hit, const float4 *sro,
     const float4 *srd, const uint32_t *target, const float4 *contrib, float4 *path_L, float4 *samp, float4 *recs,
     uint32_t *ovf, uint32_t ovf_cap, unsigned long long *stat_rows) {
@@ -1623,10 +1624,9 @@ constexpr int kMaxTraceBlocksPerCu = 8; // the traversal overflow area is sized 
 constexpr uint64_t kSampleBufferBytes = 4ull << 30;
 
 int trace_grid(const ks_device *dev, const DevScene &ds, uint32_t n, int blocks_per_cu = kMaxTraceBlocksPerCu) {
-    // 8 blocks of 256 lanes per CU keep every SIMD at 8 waves; the grid-stride loop covers the rest. The
-    // alpha-tested kernels run at 4 waves per SIMD (their opacity call needs 128 VGPRs), so 4 blocks per CU
-    // are resident and the grid stays at that.
-    const int cap = ds.alpha ? kMaxTraceBlocksPerCu / 2 : kMaxTraceBlocksPerCu;
+    // 8 blocks of 256 lanes per CU keep every SIMD at 8 waves; the grid-stride loop covers the rest. Of the
+    // alpha-tested kernels as many blocks per CU are resident as they have waves per SIMD.
+    const int cap = ds.alpha ? kAlphaTraceWaves : kMaxTraceBlocksPerCu;
     uint32_t max_blocks = (uint32_t)std::max(1, dev->n_cu) * (uint32_t)std::max(1, std::min(blocks_per_cu, cap));
     uint32_t need = (n + kTraceBlock - 1) / kTraceBlock;
     return (int)std::max(1u, std::min(max_blocks, need));

@@ -207,15 +207,13 @@ KS_DEV float hash_ray(f3 o, f3 d) {
 
 // OpacityMap::stochastic_test(uv, ro, rd) (opacity_map.cpp:20-31) for a candidate hit of triangle prim
 // at barycentric (bu, bv); the texcoord is zero where the geometry has none (compute_hit_texcoord).
-__device__ __attribute__((noinline)) bool opacity_pass(const DevScene &sc, int32_t prim, float bu, float bv, f3 o,
+KS_DEV bool opacity_pass(const DevScene &sc, int32_t prim, float bu, float bv, f3 o,
                                                        f3 d) {
     const uint4 tri = sc.tri_idx[prim];
     const DevTexMaterial &m = sc.tex_mats[sc.tex_mat_of[tri_material(tri)]];
     float u = 0.0f, v = 0.0f;
     if (geom_has_uv(sc, tri)) interp_uv(sc, tri, bu, bv, u, v);
-    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    field_eval0(tex_context(sc), m.opacity, u, v, 1, a);
-    const float op = clamp01(a[0]);
+    const float op = clamp01(field_eval0_first(tex_context(sc), m.opacity, u, v));
     if (op <= 0.0f) return false;
     if (op >= 1.0f) return true;
     return hash_ray(o, d) < op;

@@ -376,4 +376,56 @@ KS_HD void field_eval0(const TexContext &c, const DevField &f, float u, float v,
     }
 }
 
+// One channel of tex_fetch; channels the texture does not have are 0.
+KS_HD float tex_fetch1(const TexContext &c, const DevTexture &t, int x, int y, int ch) {
+    const TexLevel &l = t.lv[0];
+    const uint8_t *p = t.data + l.off + ((size_t)y * l.w + x) * t.texel_bytes;
+    if (ch < 0 || ch >= t.nc) return 0.0f;
+    if (t.dtype == kTexU8) {
+        const uint32_t b = p[ch];
+        return t.srgb ? c.luts->srgb_u8[b] : (float)b / 255.0f;
+    }
+    const float f = t.dtype == kTexU16 ? (float)((const uint16_t *)p)[ch] / 65535.0f : ((const float *)p)[ch];
+    return t.srgb ? tex_srgb_to_linear(f) : f;
+}
+
+// The first component of field_eval0, reading only the channel it takes: the traversal's opacity test. No arrays
+// indexed at run time, so nothing of it lives in scratch.
+KS_HD float field_eval0_first(const TexContext &c, const DevField &f, float u, float v) {
+    if (f.tex < 0) return f.value[0];
+    if (f.flip_v) v = 1.0f - v;
+    u = u * f.uv_scale[0] + f.uv_offset[0];
+    v = v * f.uv_scale[1] + f.uv_offset[1];
+    const DevTexture &t = c.tex[f.tex];
+    const TexLevel &l = t.lv[0];
+    const int ch = f.swizzle[0];
+    const float ut = u * (float)l.w - 0.5f, vt = v * (float)l.h - 0.5f;
+    const int iu = (int)floorf(ut), iv = (int)floorf(vt);
+    float s = 0.0f;
+    if (f.sampler == kSampNearest) {
+        s = tex_fetch1(c, t, tex_wrap(iu, l.w, f.wrap_u), tex_wrap(iv, l.h, f.wrap_v), ch);
+    } else if (f.sampler == kSampCubic) { // tex_bicubic
+        const float du = ut - (float)iu, dv = vt - (float)iv;
+        const float au[4] = {tex_dot4(f.cb, du + 1.0f), tex_dot4(f.ca, du), tex_dot4(f.ca, 1.0f - du),
+                             tex_dot4(f.cb, 2.0f - du)};
+        for (int y = 0; y < 4; ++y) {
+            const int vy = tex_wrap(iv + y - 1, l.h, f.wrap_v);
+            float cols[4];
+            for (int x = 0; x < 4; ++x) cols[x] = tex_fetch1(c, t, tex_wrap(iu + x - 1, l.w, f.wrap_u), vy, ch);
+            const float row = cols[0] * au[0] + cols[1] * au[1] + cols[2] * au[2] + cols[3] * au[3];
+            const float x = y == 0 ? dv + 1.0f : y == 1 ? dv : y == 2 ? 1.0f - dv : 2.0f - dv;
+            const float av = y == 0 || y == 3 ? tex_dot4(f.cb, x) : tex_dot4(f.ca, x);
+            s = y == 0 ? row * av : s + row * av;
+        }
+    } else { // tex_bilinear
+        const float du = ut - (float)iu, dv = vt - (float)iv;
+        const int u0 = tex_wrap(iu, l.w, f.wrap_u), v0 = tex_wrap(iv, l.h, f.wrap_v);
+        const int u1 = tex_wrap(u0 + 1, l.w, f.wrap_u), v1 = tex_wrap(v0 + 1, l.h, f.wrap_v);
+        const float w00 = (1 - du) * (1 - dv), w10 = du * (1 - dv), w01 = (1 - du) * dv, w11 = du * dv;
+        s = w00 * tex_fetch1(c, t, u0, v0, ch) + w10 * tex_fetch1(c, t, u1, v0, ch) + w01 * tex_fetch1(c, t, u0, v1, ch) +
+            w11 * tex_fetch1(c, t, u1, v1, ch);
+    }
+    return (ch >= 0 ? s : 0.0f) * f.scale[0];
+}
+
 } // namespace ksd
