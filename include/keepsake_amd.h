@@ -239,7 +239,7 @@ typedef struct ks_small_pt_params {
 #define KS_K_SHADOW 3
 #define KS_K_FILM 4
 #define KS_K_GUIDE 5
-#define KS_K_TAIL 6 /* the last paths of a render, each carried to its end by one thread */
+#define KS_K_TAIL 6 /* the last paths of a render, or all of a small one, each carried to its end by one thread */
 #define KS_K_COUNT 7
 
 typedef struct ks_render_stats {
@@ -283,7 +283,9 @@ int ks_device_set_shading(ks_device *dev, int32_t sorted);
  * them to its end in one thread instead of one wavefront iteration per bounce. Results are the same.
  * Applies to plain renders (not guided ones, not HIP-graph batches) of scenes without alpha-tested
  * triangles; 0 turns it off. Default 0: with the default 2^26-path queue the wavefront's last iterations
- * cost less than the tail kernel (40.5 against 42.0 ms for a 1080p 64-spp render). */
+ * cost less than the tail kernel (40.5 against 42.0 ms for a 1080p 64-spp render). While off, renders of
+ * at most 2^16 paths of untextured scenes are carried out by that kernel as a whole (their rays count as the
+ * wavefront's). */
 int ks_device_set_tail(ks_device *dev, int32_t max_paths);
 
 /* ---- scene: replaces create_scene + Scene::create_rtc_scene (rtcCommitScene, scene.cpp:144-160),

@@ -923,31 +923,35 @@ void k_shade(DevScene sc, RenderConsts rc, PathBufs cur, PathBufs nxt,
     wave_add_stat(stats, kNonFinite, nonfinite);
 }
 
-// The last paths of a render, each carried to its end by one thread: closest hit, shading, the NEE shadow
-// ray and the next bounce, in a loop. Once every work item has started and few paths remain, a wavefront
-// iteration costs about the time of its slowest ray, a dozen times over; here a thread waits only for its
-// own rays. The results are the wavefront's: the same traversal hits (traverse_w, the per-ray form of
+// Paths carried to their ends by one thread each: closest hit, shading, the NEE shadow ray and the next
+// bounce, in a loop. It takes the last paths of a render (once every work item has started and few paths
+// remain, a wavefront iteration costs about the time of its slowest ray, a dozen times over; here a thread
+// waits only for its own rays) and, with `whole`, all paths of a small one, whose rays are then counted as the
+// wavefront's. The results are the wavefront's: the same traversal hits (traverse_w, the per-ray form of
 // trace_rays_kind's loop), the same shading (shade_vertex), and the NEE contribution added to the path's
 // radiance, or to its sample result once the path has ended, before the next vertex, with the same
 // single addition the wavefront's traversal makes (add_nee). Plain renders of scenes without alpha-tested
-// triangles only; n paths of buffer cur, n no larger than the overflow area's lanes.
+// triangles only; the live paths of buffer cur, no more than the overflow area's lanes. Blocks of 64 to 256.
 template <int W, bool BATCH, bool TEX>
 __global__ __launch_bounds__(256) void k_tail(DevScene sc, RenderConsts rc, PathBufs cur, Queue q, float4 *samp,
-                                              uint32_t *ovf, uint32_t ovf_cap, unsigned long long *stat_rows) {
-    __shared__ uint32_t s_stack[kStackLds * 256];
-    __shared__ uint32_t s_stat[3 * 4];
+                                              uint32_t *ovf, uint32_t ovf_cap, unsigned long long *stat_rows,
+                                              uint32_t whole) {
+    __shared__ uint32_t s_stack[kStackLds * kTraceBlock];
+    __shared__ uint32_t s_cnt[8];
+    if (threadIdx.x < 8) s_cnt[threadIdx.x] = 0u;
+    __syncthreads();
     const uint32_t n = q.active();
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (blockIdx.x * blockDim.x >= n) return; // whole block idle
-    uint32_t n_rays = 0, nonfinite = 0, spills = 0;
     if (i < n) {
+        uint32_t n_closest = 0, n_shadow = 0, nonfinite = 0;
+        uint32_t n_nodes = 0, n_tris = 0, s_nodes = 0, s_tris = 0;
         TravStack st;
         st.lds = s_stack + threadIdx.x;
         st.ovf = ovf + i;
         st.ovf_stride = gridDim.x * blockDim.x;
         st.ovf_cap = ovf_cap;
         st.spills = 0;
-        uint32_t n_nodes = 0, n_tris = 0; // the tail's rays are counted, not their nodes
         const uint32_t w = cur.work[i];
         uint32_t state = cur.state[i];
         f3 beta, L;
@@ -959,7 +963,7 @@ __global__ __launch_bounds__(256) void k_tail(DevScene sc, RenderConsts rc, Path
         while (true) {
             TravHit th;
             traverse_w<false, W>(sc.nodes, sc.tris, make_trav_ray(o, d, tmin), tmax, st, th, n_nodes, n_tris);
-            ++n_rays;
+            ++n_closest;
             const float4 h = th.prim >= 0 ? make_float4(th.t, th.u, th.v, __int_as_float(th.prim))
                                           : make_float4(-1.0f, 0.0f, 0.0f, __int_as_float(-1));
             bool survive = false, shadow = false;
@@ -976,8 +980,8 @@ __global__ __launch_bounds__(256) void k_tail(DevScene sc, RenderConsts rc, Path
             if (shadow) {
                 TravHit sh;
                 const bool occluded = traverse_w<true, W>(sc.nodes, sc.tris, make_trav_ray(sh_origin, sh_dir, 0.0f),
-                                                          sh_tmax, st, sh, n_nodes, n_tris);
-                ++n_rays;
+                                                          sh_tmax, st, sh, s_nodes, s_tris);
+                ++n_shadow;
                 if (!occluded) {
                     if (survive) {
                         L.x += sh_contrib.x;
@@ -1000,11 +1004,22 @@ __global__ __launch_bounds__(256) void k_tail(DevScene sc, RenderConsts rc, Path
             tmin = 0.0f;
             tmax = kInf;
         }
-        spills = st.spills;
+        const uint32_t v[8] = {n_closest, n_shadow, n_nodes, n_tris, s_nodes, s_tris, nonfinite, st.spills};
+        for (int k = 0; k < 8; ++k)
+            if (v[k]) atomicAdd(&s_cnt[k], v[k]);
     }
-    constexpr int slots[3] = {kRaysTail, kNonFinite, kSpills};
-    const uint32_t v[3] = {n_rays, nonfinite, spills};
-    block_add_stats<4>(stat_rows, slots, v, s_stat);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long *row = stat_rows + (size_t)blockIdx.x * kStatCount;
+        if (whole) {
+            constexpr int slots[6] = {kRaysClosest, kRaysShadow, kNodesClosest, kTrisClosest, kNodesShadow, kTrisShadow};
+            for (int k = 0; k < 6; ++k) row[slots[k]] += s_cnt[k];
+        } else { // the tail's rays are counted, not their nodes
+            row[kRaysTail] += s_cnt[0] + s_cnt[1];
+        }
+        row[kNonFinite] += s_cnt[6];
+        row[kSpills] += s_cnt[7];
+    }
 }
 
 // RenderTarget2::add / add_miss (render_target.cpp:82-107) for every sample of the batch, in sample
@@ -1554,8 +1569,7 @@ template <typename... A> void launch_trace(const DevScene &ds, dim3 g, hipStream
         else hipLaunchKernelGGL((k_trace<2, false>), g, b, 0, s, ds, args...);
     }
 }
-template <typename... A> void launch_tail(const DevScene &ds, bool batch, dim3 g, hipStream_t s, A... args) {
-    const dim3 b(256);
+template <typename... A> void launch_tail(const DevScene &ds, bool batch, dim3 g, dim3 b, hipStream_t s, A... args) {
     const bool tex = ds.textured != 0;
     if (ds.width == 4) {
         if (batch) {
@@ -1782,6 +1796,14 @@ __global__ void k_capture_done(Queue q, uint32_t shadow, uint32_t *count, uint32
     *count = (uint32_t)min((uint64_t)cap, (uint64_t)*count + (shadow ? q.shadows() : q.active()));
 }
 
+// Renders of at most this many paths (untextured scenes) are carried out by one thread per path: an iteration of
+// so few rays costs the wavefront its slowest ray and its launches, and every path waits for both at each vertex.
+// With more paths the kernel's 3 waves per SIMD hold lanes of ended paths while the wavefront's stay full, and a
+// sky map lit scene is the first to lose. ms, wavefront / whole paths: Cornell 4096 paths 0.51 / 0.37, 65536 0.52 /
+// 0.36, 262144 0.61 / 0.67; room 12288 1.86 / 1.02, 61440 2.00 / 1.15, 262144 2.38 / 2.07; spheres 30000 1.89 /
+// 1.11, 65536 2.25 / 1.64; sky map 65536 1.55 / 1.49, 131072 1.57 / 1.69, 180000 1.62 / 1.81.
+constexpr uint64_t kWholePathLimit = 1u << 16;
+
 int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int max_bounces, Timer &tm,
                   ks_render_stats *stats, const GuidePass *gp = nullptr, const WavefrontOpts &wo = WavefrontOpts{}) {
     ks_device *dev = sc->dev;
@@ -1807,6 +1829,25 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
     auto trace_blocks = [&] {
         return trace_grid(dev, sc->ds, (uint32_t)(shade_blocks + shade_blocks_before) * 256u, wo.blocks_per_cu);
     };
+    // A small render, all of whose paths fit the queue at once, is two launches: ray generation, and one thread
+    // per path to its end. In blocks of 64, one wave to a CU as long as there are CUs; each block has a row of
+    // the statistics and each lane its overflow stack.
+    const unsigned whole_blocks = (unsigned)((std::min(total, kWholePathLimit) + 63) / 64);
+    if (total <= kWholePathLimit && total <= (uint64_t)Q && whole_blocks <= stat_partial_rows(dev) &&
+        whole_blocks * 64u <= ws.ovf_grid && dev->tail_paths == 0 && !gp && !wo.cap_n && !sc->ds.textured &&
+        !sc->ds.alpha) {
+        hipEvent_t e = tm.begin(KS_K_RAYGEN);
+        if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));
+        else hipLaunchKernelGGL(k_raygen<false>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));
+        tm.end(e);
+        e = tm.begin(KS_K_TAIL);
+        launch_tail(sc->ds, wo.batch, dim3(whole_blocks), dim3(64), s, rc, pb[0], view(0),
+                    ws.samp.as<float4>(), ws.ovf.as<uint32_t>(), ws.ovf_cap, stat_rows(dev), 1u);
+        tm.end(e);
+        KS_HIP(hipGetLastError());
+        if (stats) stats->iterations += 1;
+        return KS_OK;
+    }
     const bool graph = wo.graph && !gp;
     auto launch_rays = [&](int cur, uint32_t closest) {
         launch_trace(sc->ds, dim3(trace_blocks()), s, view(cur), closest, (const float4 *)pb[cur].ro,
@@ -1969,8 +2010,8 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
                     status = flush_shadow(cur); // the last shading pass's shadow rays add to these paths
                     if (status) break;
                     hipEvent_t e = tm.begin(KS_K_TAIL);
-                    launch_tail(sc->ds, wo.batch, dim3((unsigned)((c.paths + 255) / 256)), s, rc, pb[cur], view(cur),
-                                ws.samp.as<float4>(), ws.ovf.as<uint32_t>(), ws.ovf_cap, stat_rows(dev));
+                    launch_tail(sc->ds, wo.batch, dim3((unsigned)((c.paths + 255) / 256)), dim3(256), s, rc, pb[cur],
+                                view(cur), ws.samp.as<float4>(), ws.ovf.as<uint32_t>(), ws.ovf_cap, stat_rows(dev), 0u);
                     tm.end(e);
                     KS_HIP(hipGetLastError());
                     tail_ran = true;

@@ -32,3 +32,28 @@ def test_known_and_read_ends_agree(ks, device, cornell, bounces, size, spp):
     assert wts.sum() == w * h * spp
     for (r, g), c, s in out[1:]:
         assert np.array_equal(r, rgb) and np.array_equal(g, wts) and (c, s) == (rc, rs)
+
+
+@pytest.mark.parametrize("name,seed", [("cornell", 0), ("spheres_small", 1)])
+@pytest.mark.parametrize("w,h,spp", [(64, 1, 1), (65, 1, 1), (512, 128, 1), (331, 99, 2), (331, 33, 5), (513, 128, 1)])
+def test_whole_paths_equal_the_wavefront(ks, device, name, seed, w, h, spp):
+    """Up to 2^16 paths, one thread per path; just above, and with a queue that cannot hold them, the wavefront."""
+    print("whole paths", name, w, h, spp, flush=True)
+    hs = ks.procedural_scene(name, seed)
+    sc = ks.Scene(device, hs)
+    cam = dict(hs.camera)
+    cam["aspect"] = w / h
+    out = []
+    for queue in (0, max(256, w * h * spp // 3)):
+        film = ks.Film(device, w, h)
+        p = ks.small_pt_params(bounces=9, render_width=w, render_height=h, spp=spp, spp_prog_interval=spp, rng_seed=3,
+                               queue_size=queue)
+        st = ks.small_pt_render(sc, cam, p, film)
+        out.append((film.download(), st))
+        film.close()
+    sc.close()
+    ((a, wa), sa), ((b, wb), sb) = out
+    print("iterations", sa["iterations"], sb["iterations"], flush=True)
+    assert np.array_equal(a, b) and np.array_equal(wa, wb)
+    for k in ("rays_closest", "rays_shadow", "rays_tail", "paths", "nonfinite"):
+        assert sa[k] == sb[k], k
