@@ -381,21 +381,26 @@ KS_DEV uint32_t visit_node(const float4 *__restrict__ nodes, const TravRay &r, f
     return st.pop();
 }
 
-// Rays first, first + stride, ... < n on one lane, with replacement: a lane whose ray has finished
-// stores its result and loads its next ray at once, while the other lanes of the wave go on with
-// theirs. The wave then never waits for its slowest ray before fetching more work. Leaves are found
+// Rays first, first + stride, ... < n on one lane. Leaves are found
 // speculatively: a lane that reaches a leaf sets it aside and keeps visiting inner nodes until every
 // lane of the wave holds a leaf (or has none left), and then all lanes test their leaves together
-// (the persistent speculative while-while loop of Aila and Laine, HPG 2009). A lane may set aside a
+// (the speculative while-while loop of Aila and Laine, HPG 2009). A lane may set aside a
 // second leaf while it waits, rather than idle on it (measured: traversal 29.7 -> 28.5 ms per 1080p
 // render); its triangles are tested after the first leaf's, in traversal order. The inner-node loop
 // also ends early when few lanes are still searching and some lane has finished, so that finished
-// lanes do not idle through the others' searches before they take a new ray. Each ray's closest hit is
+// lanes do not idle through the others' searches. Each ray's closest hit is
 // the one traverse_w gives; among triangles hit at exactly the same t, the first one tested wins.
 // load(i, ray) fills the ray and returns its tmax; store(i, hit) takes the result (prim < 0: miss).
 // With ALPHA, a triangle whose record carries a non-zero v1.w is an alpha-tested candidate: filter(prim,
 // u, v, ray) decides whether the hit counts (Embree's intersection filter, scene.cpp:175-204). A hit it
 // rejects is skipped and traversal goes on, for closest and any hits alike.
+// When lanes take their next rays: without REPLACE the wave's rays end together (the compiled loop holds the lanes
+// whose rays have ended until all have). With REPLACE a lane takes its next ray at once, unless together(i) says
+// that ray i is one of neighbours that stay together. Replacement pays where the rays of a wave differ in length
+// and each visit costs much: the alpha-tested traversal of a foliage scene, 7.55 ms per render together, 6.77 with 16
+// lanes waiting before they are served, 6.39 with 4, 6.30 at once. It costs where neighbours visit the same nodes:
+// plain scenes lose that with it, 28.2 -> 42 ms for a 1080p sphere field (also when camera rays stay together; a
+// room scene 9.25 -> 8.97).
 struct NoFilter {
     KS_DEV bool operator()(int32_t, float, float, const TravRay &) const { return true; }
 };
@@ -406,30 +411,47 @@ template <bool ANY> struct FixedKind {
     KS_DEV bool operator()(uint32_t) const { return ANY; }
 };
 
-template <int W, bool ALPHA = false, typename Kind, typename Load, typename Store, typename Filter = NoFilter>
+template <int W, bool ALPHA, bool REPLACE, typename Kind, typename Load, typename Store, typename Filter,
+          typename Together>
 KS_DEV void trace_rays_kind(const float4 *__restrict__ nodes, const float4 *__restrict__ tris, uint32_t i, uint32_t n,
                             uint32_t stride, TravStack &st, Kind any_hit, Load &&load, Store &&store,
-                            uint32_t &n_nodes, uint32_t &n_tris, uint32_t &n_rays, Filter filter = Filter()) {
+                            uint32_t &n_nodes, uint32_t &n_tris, uint32_t &n_rays, Filter filter, Together together) {
     if (i >= n) return;
     TravRay r;
     TravHit hit;
     float tmax = load(i, r);
     hit.prim = -1;
     st.sp = 0;
+    bool finished = false;   // REPLACE: the ray has ended; its result is stored with the next refill
     uint32_t node = 0;       // next node to visit (valid while !exhausted)
     uint32_t leaf = 0;       // leaf set aside for testing (0: none; leaves carry kLeafBit)
     uint32_t leaf2 = 0;      // a second leaf set aside while the first waits
     bool exhausted = false;  // no node left to visit for this ray
     while (true) {
+        if constexpr (REPLACE) {
+            if (!__any(!finished) || (__any(finished) && !__any(together(i)))) {
+                if (finished) {
+                    store(i, hit);
+                    ++n_rays;
+                    i += stride;
+                    if (i >= n) break;
+                    tmax = load(i, r);
+                    hit.prim = -1;
+                    st.sp = 0;
+                    node = 0;
+                    finished = false;
+                }
+            }
+        }
         // inner nodes, until every lane of the wave holds a leaf or has nothing left to visit
         while (true) {
-            if (!exhausted && (node & kLeafBit) == 0) {
+            if (!finished && !exhausted && (node & kLeafBit) == 0) {
                 ++n_nodes;
                 bool empty = false;
                 node = visit_node<W>(nodes, r, tmax, st, node, empty);
                 exhausted = empty;
             }
-            if (!exhausted && (node & kLeafBit) != 0 && leaf2 == 0) {
+            if (!finished && !exhausted && (node & kLeafBit) != 0 && leaf2 == 0) {
                 if (leaf == 0) leaf = node;
                 else leaf2 = node;
                 if (st.sp == 0) exhausted = true;
@@ -438,7 +460,7 @@ KS_DEV void trace_rays_kind(const float4 *__restrict__ nodes, const float4 *__re
             // leave for the leaf tests when no lane is left without a leaf, or, so that finished lanes
             // take new rays sooner, when fewer than kTraverseBusyMin lanes are still looking for one while
             // some lane has finished its ray
-            const uint64_t busy = __ballot(leaf == 0 && !exhausted);
+            const uint64_t busy = __ballot(!finished && leaf == 0 && !exhausted);
             if (busy == 0) break;
             if (__popcll(busy) < kTraverseBusyMin && __any(exhausted)) break;
         }
@@ -515,7 +537,12 @@ KS_DEV void trace_rays_kind(const float4 *__restrict__ nodes, const float4 *__re
                 }
             }
         }
-        if (done || exhausted) {
+        if constexpr (REPLACE) {
+            if (done || exhausted) {
+                finished = true;
+                exhausted = false;
+            }
+        } else if (done || exhausted) {
             store(i, hit);
             ++n_rays;
             i += stride;
@@ -535,8 +562,8 @@ template <bool ANY, int W, bool ALPHA = false, typename Load, typename Store, ty
 KS_DEV void trace_rays(const float4 *__restrict__ nodes, const float4 *__restrict__ tris, uint32_t i, uint32_t n,
                        uint32_t stride, TravStack &st, Load &&load, Store &&store, uint32_t &n_nodes,
                        uint32_t &n_tris, uint32_t &n_rays, Filter filter = Filter()) {
-    trace_rays_kind<W, ALPHA>(nodes, tris, i, n, stride, st, FixedKind<ANY>(), load, store, n_nodes, n_tris, n_rays,
-                              filter);
+    trace_rays_kind<W, ALPHA, false>(nodes, tris, i, n, stride, st, FixedKind<ANY>(), load, store, n_nodes, n_tris,
+                                     n_rays, filter, [](uint32_t) { return true; });
 }
 
 // Dispatch on the node width of the scene (2 or 4).

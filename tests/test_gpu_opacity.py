@@ -63,3 +63,35 @@ def test_opacity_fields_match_oracle(ks, device, ora, sampler, dtype, srgb, chan
     assert (g == r).mean() > 0.999
     assert (sc.occluded(rays).astype(bool) == (g >= 0)).mean() > 0.999
     sc.close()
+
+
+@pytest.mark.parametrize("w,h,spp", [(63, 1, 1), (97, 61, 3), (500, 300, 8)])
+@pytest.mark.parametrize("branching", [4, 2])
+def test_ray_replacement_does_not_change_a_render(ks, device, w, h, spp, branching):
+    """Alpha-tested path launches mix camera rays, which stay together, with later rays, which are replaced at
+    once; the mix and the lane a ray falls to depend on the queue. The films and ray counts must not."""
+    print("replacement", w, h, spp, branching, flush=True)
+    import sys
+    from pathlib import Path
+
+    sys.path.insert(0, str(Path(__file__).parent))
+    from texture_scenes import textured_box
+
+    hs = textured_box()
+    sc = ks.Scene(device, hs, bvh={"branching": branching})
+    cam = dict(hs.camera)
+    cam["aspect"] = w / h
+    out = []
+    for queue in (0, 256 if w * h * spp < 20000 else 65536, max(256, w * h * spp * 2 // 3)):
+        film = ks.Film(device, w, h)
+        p = ks.small_pt_params(bounces=7, render_width=w, render_height=h, spp=spp, spp_prog_interval=spp,
+                               rng_seed=5, queue_size=queue)
+        st = ks.small_pt_render(sc, cam, p, film)
+        out.append((film.download(), st))
+        film.close()
+    sc.close()
+    (a, wa), sa = out[0]
+    for (b, wb), sb in out[1:]:
+        assert np.array_equal(a, b) and np.array_equal(wa, wb)
+        for k in ("rays_closest", "rays_shadow", "paths", "nonfinite"):
+            assert sa[k] == sb[k], k
