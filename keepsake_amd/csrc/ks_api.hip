@@ -1059,6 +1059,9 @@ __global__ __launch_bounds__(256) void k_film(RenderConsts rc, const float4 *sam
 // Film fold of a batched chunk: one thread per (segment, pixel of its view's crop); thread_base[k] is the
 // first thread of segment k, seg_items[k] its item count. Samples are folded in sample order, so every
 // view's film is the same as a render of that view alone.
+// Bound by memory: a pixel's samples lie together, so a wave's loads touch 64 lines each. Eight samples, a 128-byte
+// line, are loaded together; one at a time the lines left the L1 before their next sample was read (41 M samples of
+// 12 views: 951 us one at a time, 259 with eight).
 __global__ __launch_bounds__(256) void k_film_batch(const RenderConsts *views, const uint4 *segs,
                                                     const uint32_t *thread_base, const uint32_t *seg_items, int n_segs,
                                                     uint32_t n_threads, const float4 *samp, double *const *rgbs,
@@ -1080,8 +1083,8 @@ __global__ __launch_bounds__(256) void k_film_batch(const RenderConsts *views, c
     double *rgb = rgbs[sg.y], *wts = wtss[sg.y];
     double r = rgb[3 * px], g = rgb[3 * px + 1], b = rgb[3 * px + 2];
     double wh = wts[2 * px], wm = wts[2 * px + 1];
-    for (uint32_t k = 0; k < nb; ++k) {
-        float4 v4 = samp[(size_t)sg.x + (size_t)p * nb + k];
+    const float4 *sp = samp + (size_t)sg.x + (size_t)p * nb;
+    auto fold = [&](float4 v4) {
         if (v4.w != 0.0f) {
             wh += 1.0;
             r += (double)v4.x;
@@ -1090,7 +1093,16 @@ __global__ __launch_bounds__(256) void k_film_batch(const RenderConsts *views, c
         } else {
             wm += 1.0;
         }
+    };
+    uint32_t k = 0;
+    for (; k + 8 <= nb; k += 8) {
+        float4 v8[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v8[j] = sp[k + j];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) fold(v8[j]);
     }
+    for (; k < nb; ++k) fold(sp[k]);
     rgb[3 * px] = r;
     rgb[3 * px + 1] = g;
     rgb[3 * px + 2] = b;

@@ -84,3 +84,21 @@ def test_views_split_across_chunks(ks, device, cornell, graph):
     for f in films:
         f.close()
     sc.close()
+
+
+def test_batch_folds_every_remainder_of_eight(ks, device, cornell):
+    """The film fold reads eight samples of a pixel at a time, then the rest one by one."""
+    sc = ks.Scene(device, cornell)
+    views = [ks.small_pt_params(bounces=4, render_width=37, render_height=5, spp=n, spp_prog_interval=n, rng_seed=n)
+             for n in (1, 7, 8, 9, 15, 16, 17, 23)]
+    films = [ks.Film(device, 37, 5) for _ in views]
+    ks.small_pt_render_batch(sc, [(cornell.camera, p, f) for p, f in zip(views, films)])
+    for p, f in zip(views, films):
+        alone = ks.Film(device, 37, 5)
+        ks.small_pt_render(sc, cornell.camera, p, alone)
+        a, wa = f.download()
+        b, wb = alone.download()
+        alone.close()
+        f.close()
+        assert np.array_equal(a, b) and np.array_equal(wa, wb)
+    sc.close()
