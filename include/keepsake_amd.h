@@ -275,17 +275,19 @@ int ks_device_set_timing(ks_device *dev, int32_t enable);
 /* Shading order of the wavefront (no counterpart in the reference, whose CPU loop shades one path at a time,
  * Material::sample_with_nee, material.cpp:101-167): 0 (default) shades every path with one kernel; 1 sorts
  * each bounce's paths by material class (escaped rays, opaque dielectrics, metals, other materials) and
- * shades each class with a kernel compiled for its BSDF lobes. Results are the same either way; textured
- * scenes always use one kernel. */
+ * shades each class with a kernel compiled for its BSDF lobes. Results agree up to the rounding of a few
+ * GGX terms (over 99% of pixels are equal bit for bit); textured scenes always use one kernel. With 1, small
+ * renders run the wavefront too (see ks_device_set_tail). */
 int ks_device_set_shading(ks_device *dev, int32_t sorted);
 /* The end of a render's wavefront (no counterpart in the reference, whose CPU loop traces each path to its
  * end): once every work item has started and at most max_paths paths remain, one kernel carries each of
  * them to its end in one thread instead of one wavefront iteration per bounce. Results are the same.
  * Applies to plain renders (not guided ones, not HIP-graph batches) of scenes without alpha-tested
  * triangles; 0 turns it off. Default 0: with the default 2^26-path queue the wavefront's last iterations
- * cost less than the tail kernel (40.5 against 42.0 ms for a 1080p 64-spp render). While off, renders of
- * at most 2^16 paths of untextured scenes are carried out by that kernel as a whole (their rays count as the
- * wavefront's). */
+ * cost less than the tail kernel (40.5 against 42.0 ms for a 1080p 64-spp render). While off, plain and
+ * batched renders of at most 2^16 paths of untextured scenes, whose paths all fit the queue, are carried out by
+ * that kernel as a whole (their rays count as the wavefront's, and queue size and traversal blocks do not
+ * matter). Any other value, even 1, and sorted shading send small renders through the wavefront. */
 int ks_device_set_tail(ks_device *dev, int32_t max_paths);
 
 /* ---- scene: replaces create_scene + Scene::create_rtc_scene (rtcCommitScene, scene.cpp:144-160),

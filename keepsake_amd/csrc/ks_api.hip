@@ -1848,10 +1848,11 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
     };
     // A small render, all of whose paths fit the queue at once, is two launches: ray generation, and one thread
     // per path to its end. In blocks of 64, one wave to a CU as long as there are CUs; each block has a row of
-    // the statistics and each lane its overflow stack.
+    // the statistics and each lane its overflow stack. Sorted shading has kernels of its own (their rounding
+    // differs in a few GGX terms), so a sorted render keeps to them whatever its chunks' sizes.
     const unsigned whole_blocks = (unsigned)((std::min(total, kWholePathLimit) + 63) / 64);
     if (total <= kWholePathLimit && total <= (uint64_t)Q && whole_blocks <= stat_partial_rows(dev) &&
-        whole_blocks * 64u <= ws.ovf_grid && dev->tail_paths == 0 && !gp && !wo.cap_n && !sc->ds.textured &&
+        whole_blocks * 64u <= ws.ovf_grid && dev->tail_paths == 0 && !sorted && !gp && !wo.cap_n && !sc->ds.textured &&
         !sc->ds.alpha) {
         hipEvent_t e = tm.begin(KS_K_RAYGEN);
         if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));

@@ -75,3 +75,27 @@ def test_sorted_shading_guided_and_batched(ks, device, cornell):
     # miss) weights, which the camera rays decide, are compared
     assert np.array_equal(res[0][1], res[1][1]) and res[0][1][..., 0].sum() > 0
     sc.close()
+
+
+@pytest.mark.parametrize("name,seed", [("cornell", 0), ("spheres_small", 1)])
+def test_small_sorted_renders_keep_their_kernels(ks, device, name, seed):
+    """A sorted render of few paths runs the wavefront and its class kernels, so its film does not depend on
+    whether the queue holds all of them."""
+    hs = ks.procedural_scene(name, seed)
+    sc = ks.Scene(device, hs)
+    W, H = 96, 64
+    cam = dict(hs.camera)
+    cam["aspect"] = W / H
+    out = []
+    device.set_shading(True)
+    for queue in (0, 4096):
+        f = ks.Film(device, W, H)
+        p = ks.small_pt_params(bounces=9, render_width=W, render_height=H, spp=4, spp_prog_interval=4, queue_size=queue)
+        out.append((ks.small_pt_render(sc, cam, p, f), f.download()))
+        f.close()
+    device.set_shading(False)  # the default
+    (sa, (a, wa)), (sb, (b, wb)) = out
+    print(name, "iterations", sa["iterations"], sb["iterations"], flush=True)
+    assert sa["iterations"] == 10 and sb["iterations"] >= 10 and sa["launches"]["tail"] == 0
+    assert np.array_equal(wa, wb) and np.array_equal(a, b)
+    sc.close()
