@@ -96,6 +96,8 @@ def test_small_sorted_renders_keep_their_kernels(ks, device, name, seed):
     device.set_shading(False)  # the default
     (sa, (a, wa)), (sb, (b, wb)) = out
     print(name, "iterations", sa["iterations"], sb["iterations"], flush=True)
-    assert sa["iterations"] == 10 and sb["iterations"] >= 10 and sa["launches"]["tail"] == 0
+    # more than the one of whole paths; at most one for each of the ten vertices of the longest path that the bounces
+    # allow, fewer where a control read finds every path ended
+    assert 1 < sa["iterations"] <= 10 and sb["iterations"] > 1 and sa["launches"]["tail"] == 0
     assert np.array_equal(wa, wb) and np.array_equal(a, b)
     sc.close()
