@@ -1788,6 +1788,7 @@ struct WavefrontOpts {
     bool batch = false;
     bool graph = false;
     int blocks_per_cu = kMaxTraceBlocksPerCu;
+    bool whole_paths = true; // a small run may be carried out by one thread per path (runs_whole_paths)
     // ray capture (eager launches only): every closest-hit and shadow ray of the run, appended as
     // (o, tmin), (d, tmax) pairs to cap_c / cap_s up to cap_max each; cap_n[0], cap_n[1] count them
     float4 *cap_c = nullptr, *cap_s = nullptr;
@@ -1821,6 +1822,17 @@ __global__ void k_capture_done(Queue q, uint32_t shadow, uint32_t *count, uint32
 // 1.11, 65536 2.25 / 1.64; sky map 65536 1.55 / 1.49, 131072 1.57 / 1.69, 180000 1.62 / 1.81.
 constexpr uint64_t kWholePathLimit = 1u << 16;
 
+// Whether a run of `total` paths through a queue of Q is carried out by one thread per path, in blocks of 64, one
+// wave to a CU as long as there are CUs. Each block needs a row of the statistics; its lanes then have their
+// overflow stacks too, as the overflow area holds kTraceBlock lanes for each row. Sorted shading has kernels of
+// its own (their rounding differs in a few GGX terms), so a sorted render keeps to them whatever its chunks' sizes.
+bool runs_whole_paths(const ks_scene *sc, uint64_t total, uint32_t Q, bool guided, const WavefrontOpts &wo) {
+    const ks_device *dev = sc->dev;
+    return wo.whole_paths && total <= kWholePathLimit && total <= (uint64_t)Q &&
+           (total + 63) / 64 <= stat_partial_rows(dev) && dev->tail_paths == 0 && !dev->sorted_shading && !guided &&
+           !wo.cap_n && !sc->ds.textured && !sc->ds.alpha;
+}
+
 int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int max_bounces, Timer &tm,
                   ks_render_stats *stats, const GuidePass *gp = nullptr, const WavefrontOpts &wo = WavefrontOpts{}) {
     ks_device *dev = sc->dev;
@@ -1846,14 +1858,9 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
     auto trace_blocks = [&] {
         return trace_grid(dev, sc->ds, (uint32_t)(shade_blocks + shade_blocks_before) * 256u, wo.blocks_per_cu);
     };
-    // A small render, all of whose paths fit the queue at once, is two launches: ray generation, and one thread
-    // per path to its end. In blocks of 64, one wave to a CU as long as there are CUs; each block has a row of
-    // the statistics and each lane its overflow stack. Sorted shading has kernels of its own (their rounding
-    // differs in a few GGX terms), so a sorted render keeps to them whatever its chunks' sizes.
-    const unsigned whole_blocks = (unsigned)((std::min(total, kWholePathLimit) + 63) / 64);
-    if (total <= kWholePathLimit && total <= (uint64_t)Q && whole_blocks <= stat_partial_rows(dev) &&
-        whole_blocks * 64u <= ws.ovf_grid && dev->tail_paths == 0 && !sorted && !gp && !wo.cap_n && !sc->ds.textured &&
-        !sc->ds.alpha) {
+    // A small render is two launches: ray generation, and one thread per path to its end.
+    if (runs_whole_paths(sc, total, Q, gp != nullptr, wo)) {
+        const unsigned whole_blocks = (unsigned)((total + 63) / 64);
         hipEvent_t e = tm.begin(KS_K_RAYGEN);
         if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));
         else hipLaunchKernelGGL(k_raygen<false>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));
@@ -3351,10 +3358,15 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
         wo.graph = o.disable_graph == 0;
         uint32_t Q = 0;
         // autotuner: queue size 2^18..2^25 x traversal blocks per CU {4, 8}, timed on the first chunk's first
-        // items (at most 2^25), cached per scene and workload size
+        // items (at most 2^25), cached per scene and workload size. Both are the wavefront's settings: a batch whose
+        // every chunk is carried out by one thread per path has nothing to tune, and the probes of the others
+        // run the wavefront however small they are.
+        const uint32_t small_q = (uint32_t)std::max<uint64_t>(std::min<uint64_t>(max_items, kWholePathLimit), 256);
         if (o.queue_size > 0) {
             Q = (uint32_t)std::min<int64_t>(o.queue_size, 1 << 26);
             wo.blocks_per_cu = o.trace_blocks_per_cu > 0 ? o.trace_blocks_per_cu : kMaxTraceBlocksPerCu;
+        } else if (runs_whole_paths(scene, max_items, small_q, false, wo)) {
+            Q = small_q;
         } else if (dev->tune_scene == scene && dev->tune_items == paths) {
             Q = dev->tune_q;
             wo.blocks_per_cu = dev->tune_bpc;
@@ -3385,6 +3397,7 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
                     if (e) return e;
                     WavefrontOpts pw = wo;
                     pw.blocks_per_cu = bpc;
+                    pw.whole_paths = false;
                     Timer ptm{dev};
                     int saved = dev->timing;
                     dev->timing = 0;

@@ -102,3 +102,30 @@ def test_batch_folds_every_remainder_of_eight(ks, device, cornell):
         f.close()
         assert np.array_equal(a, b) and np.array_equal(wa, wb)
     sc.close()
+
+
+def test_small_batches_are_not_tuned(ks, device, cornell):
+    """Queue size and traversal blocks are the wavefront's settings: a batch carried out by one thread per path is
+    not timed over them and reports the defaults, whichever probe would have been the fastest. Chunks of both
+    kinds in one batch give the films of single renders."""
+    sc = ks.Scene(device, cornell)
+    for n in range(1, 9):
+        film = ks.Film(device, 32, 32)
+        p = ks.small_pt_params(bounces=4, render_width=32, render_height=32, spp=n, spp_prog_interval=n)
+        st = ks.small_pt_render_batch(sc, [(cornell.camera, p, film)])
+        assert (st["iterations"], st["queue_size"], st["trace_blocks_per_cu"]) == (1, 1024 * n, 8)
+        film.close()
+    sizes = [(32, 32, 4), (512, 384, 1), (40, 20, 3)]  # chunks of 4096, 196 608 and 2400 items
+    films = [ks.Film(device, w, h) for w, h, _ in sizes]
+    params = [ks.small_pt_params(bounces=4, render_width=w, render_height=h, spp=n, spp_prog_interval=n)
+              for w, h, n in sizes]
+    st = ks.small_pt_render_batch(sc, [(cornell.camera, p, f) for p, f in zip(params, films)], max_chunk_items=197_000)
+    print("chunks", st["batch_chunks"], "iterations", st["iterations"], "queue", st["queue_size"], flush=True)
+    assert st["batch_chunks"] == 3 and st["iterations"] > 5
+    for p, f in zip(params, films):
+        alone = ks.Film(device, f.width, f.height)
+        ks.small_pt_render(sc, cornell.camera, p, alone)
+        assert all(np.array_equal(a, b) for a, b in zip(f.download(), alone.download()))
+        alone.close()
+        f.close()
+    sc.close()
