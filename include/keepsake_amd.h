@@ -244,7 +244,8 @@ typedef struct ks_small_pt_params {
 
 typedef struct ks_render_stats {
     double wall_ms;                     /* host wall time of the render call */
-    double kernel_ms[KS_K_COUNT];       /* summed event time per kernel class (0 unless timing on) */
+    double kernel_ms[KS_K_COUNT];       /* summed event time per kernel class (0 unless timing on). Batches with
+                                           a HIP graph neither time nor count ray generation, traversal and shading */
     uint64_t launches[KS_K_COUNT];
     uint64_t paths;                     /* camera samples traced (W*H*spp over the crop) */
     uint64_t rays_closest;              /* primary + extension rays of the wavefront's traversal kernel */

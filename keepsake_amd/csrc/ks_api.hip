@@ -1858,10 +1858,11 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
     auto trace_blocks = [&] {
         return trace_grid(dev, sc->ds, (uint32_t)(shade_blocks + shade_blocks_before) * 256u, wo.blocks_per_cu);
     };
+    const bool graph = wo.graph && !gp;
     // A small render is two launches: ray generation, and one thread per path to its end.
     if (runs_whole_paths(sc, total, Q, gp != nullptr, wo)) {
         const unsigned whole_blocks = (unsigned)((total + 63) / 64);
-        hipEvent_t e = tm.begin(KS_K_RAYGEN);
+        hipEvent_t e = graph ? nullptr : tm.begin(KS_K_RAYGEN);
         if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));
         else hipLaunchKernelGGL(k_raygen<false>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));
         tm.end(e);
@@ -1873,7 +1874,6 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
         if (stats) stats->iterations += 1;
         return KS_OK;
     }
-    const bool graph = wo.graph && !gp;
     auto launch_rays = [&](int cur, uint32_t closest) {
         launch_trace(sc->ds, dim3(trace_blocks()), s, view(cur), closest, (const float4 *)pb[cur].ro,
                      (const float4 *)pb[cur].rd, ws.hit.as<float4>(), (const float4 *)ws.sh_o.as<float4>(),
@@ -1881,7 +1881,8 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
                      (const float4 *)ws.sh_c.as<float4>(), pb[cur].L, ws.samp.as<float4>(),
                      gp ? gp->shade.recs : (float4 *)nullptr, ws.ovf.as<uint32_t>(), ws.ovf_cap, stat_rows(dev));
     };
-    // One iteration reading buffer cur and writing buffer 1 - cur; no events while a graph is captured.
+    // One iteration reading buffer cur and writing buffer 1 - cur. Replayed iterations cannot record events, so
+    // with a graph none of them does: the kernel times of the eager ones alone would be a part of the total.
     // Its traversal also traces the previous shading pass's shadow rays (k_trace): their contributions go
     // to the survivors' slots of buffer cur (ray generation fills the slots after them) and to per-sample
     // results, before this iteration's shading reads the slots and refills the shadow queue.
@@ -1891,12 +1892,11 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
     // beyond last_gen + max bounce have no guided vertex and skip the inference.
     int iter_index = 0;
     int last_gen = total <= (uint64_t)Q ? 0 : -1; // -1: not known yet
-    bool capturing = false;
     auto iteration = [&](int cur) -> int {
         const Queue q = view(cur);
         hipEvent_t e = nullptr;
         if (gen_blocks > 0) {
-            e = capturing ? nullptr : tm.begin(KS_K_RAYGEN);
+            e = graph ? nullptr : tm.begin(KS_K_RAYGEN);
             if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[cur], q);
             else hipLaunchKernelGGL(k_raygen<false>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[cur], q);
             tm.end(e);
@@ -1909,7 +1909,7 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
                                (const float4 *)ws.sh_d.as<float4>(), wo.cap_s, wo.cap_n + 1, wo.cap_max);
             hipLaunchKernelGGL(k_capture_done, dim3(1), dim3(1), 0, s, q, 1u, wo.cap_n + 1, wo.cap_max);
         }
-        e = capturing ? nullptr : tm.begin(KS_K_CLOSEST);
+        e = graph ? nullptr : tm.begin(KS_K_CLOSEST);
         launch_rays(cur, 1u);
         tm.end(e);
         auto young = [&](int b) { return last_gen < 0 || iter_index - last_gen < b; };
@@ -1925,7 +1925,7 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
             tm.end(e);
             if (ge) return ge;
         }
-        e = capturing ? nullptr : tm.begin(KS_K_SHADE);
+        e = graph ? nullptr : tm.begin(KS_K_SHADE);
         if (sorted)
             hipLaunchKernelGGL(k_classify, dim3(tblocks), dim3(256), 0, s, sc->ds, (const float4 *)ws.hit.as<float4>(), q,
                                ws.order.as<uint32_t>(), Q);
@@ -1955,10 +1955,8 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
     hipGraph_t g = nullptr;
     if (graph) {
         KS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        capturing = true;
         int e0 = iteration(0);
         int e1 = iteration(1);
-        capturing = false;
         hipError_t ce = hipStreamEndCapture(s, &g);
         if (e0 || e1) {
             if (g) (void)hipGraphDestroy(g);

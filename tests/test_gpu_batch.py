@@ -129,3 +129,26 @@ def test_small_batches_are_not_tuned(ks, device, cornell):
         alone.close()
         f.close()
     sc.close()
+
+
+@pytest.mark.parametrize("queue", [1 << 13, 1 << 17])
+def test_kernel_times_of_a_graph_batch_are_none_or_whole(ks, device, cornell, queue):
+    """Replayed iterations record no events, so no iteration of a graph batch does, nor its small last chunk (9600
+    items, one thread per path); eagerly launched, every class that ran is timed."""
+    sc = ks.Scene(device, cornell)
+    film = ks.Film(device, 160, 120)
+    p = ks.small_pt_params(bounces=8, render_width=160, render_height=120, spp=8, spp_prog_interval=8)
+    small = ks.Film(device, 160, 60)
+    q = ks.small_pt_params(bounces=8, render_width=160, render_height=60, spp=1, spp_prog_interval=1)
+    device.set_timing(True)
+    st = {g: ks.small_pt_render_batch(sc, [(cornell.camera, p, film), (cornell.camera, q, small)], queue_size=queue,
+                                      graph=g, max_chunk_items=160 * 120 * 8) for g in (True, False)}
+    device.set_timing(False)
+    film.close()
+    small.close()
+    sc.close()
+    print(queue, st[True]["kernel_ms"], st[True]["launches"], st[False]["kernel_ms"], flush=True)
+    for k in ("raygen", "closest", "shade"):
+        assert st[True]["kernel_ms"][k] == 0 and st[True]["launches"][k] == 0
+        assert st[False]["kernel_ms"][k] > 0 and st[False]["launches"][k] > 0
+    assert st[True]["kernel_ms"]["film"] > 0 and st[True]["batch_chunks"] == 2
