@@ -200,10 +200,16 @@ KS_DEV float head_backward(const float o[kGuideOut], f3 wi, float c, float g[kGu
 // ---------------------------------------------------------------------------------------------------
 // Hash-grid encoding (multiresolution, trilinear, FP16 features)
 // ---------------------------------------------------------------------------------------------------
+// Whether a level of this resolution is stored densely, i.e. its (res + 1)^3 corners fit the table. Tables have at
+// most 2^24 = 256^3 entries, so only resolutions below 256 can, and their cube fits 32 bits (that of any resolution
+// does not fit 64: (2^22)^3 wraps to 0).
+__host__ __device__ constexpr bool grid_dense(uint32_t res, uint32_t log2_T) {
+    return res < 256u && (res + 1u) * (res + 1u) * (res + 1u) <= (1u << log2_T);
+}
+
 KS_DEV uint32_t grid_index(uint32_t x, uint32_t y, uint32_t z, uint32_t res, uint32_t log2_T) {
-    uint32_t T = 1u << log2_T;
-    uint64_t side = (uint64_t)res + 1;
-    if (side * side * side <= T) return x + (uint32_t)side * (y + (uint32_t)side * z); // dense level
+    const uint32_t T = 1u << log2_T, side = res + 1u;
+    if (grid_dense(res, log2_T)) return x + side * (y + side * z);
     return (x ^ (y * 2654435761u) ^ (z * 805459861u)) & (T - 1u);
 }
 

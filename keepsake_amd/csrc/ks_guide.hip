@@ -1262,6 +1262,7 @@ int ks_guide_create(ks_device *dev, const ks_guide_config *cfg_in, const float b
         if (c.weight_clamp == 0.0f) c.weight_clamp = 20.0f;
         KS_REQUIRE(c.log2_table_size >= 10 && c.log2_table_size <= 24, "log2_table_size must be in [10, 24]");
         KS_REQUIRE(c.max_resolution >= c.base_resolution && c.base_resolution >= 2.0f, "bad grid resolutions");
+        KS_REQUIRE(c.max_resolution < 0x1p32f, "max_resolution must be below 2^32"); // levels hold 32-bit ones
         KS_REQUIRE(c.guide_fraction >= 0.0f && c.guide_fraction < 1.0f, "guide_fraction must be in [0, 1)");
         KS_REQUIRE(c.train_spp >= 0, "train_spp must be non-negative");
         g->cfg = c;
@@ -1293,10 +1294,10 @@ int ks_guide_create(ks_device *dev, const ks_guide_config *cfg_in, const float b
             // of kScatterEntries. Entries past a dense level's are never touched; their gradient stays zero.
             std::vector<uint4> tiles;
             for (int l = 0; l < kGuideLevels; ++l) {
-                const uint64_t side = (uint64_t)g->res[l] + 1, dense = side * side * side, T = 1ull << g->log2_T;
-                const uint32_t used = (uint32_t)std::min(dense, T);
+                const bool dense = grid_dense(g->res[l], g->log2_T);
+                const uint32_t side = g->res[l] + 1u, used = dense ? side * side * side : 1u << g->log2_T;
                 const uint32_t n = (used + kScatterEntries - 1) / kScatterEntries;
-                const uint32_t shares = std::max(1u, (dense <= T ? kScatterDenseShares : kScatterShares) / n);
+                const uint32_t shares = std::max(1u, (dense ? kScatterDenseShares : kScatterShares) / n);
                 for (uint32_t e = 0; e < used; e += kScatterEntries)
                     for (uint32_t k = 0; k < shares; ++k)
                         tiles.push_back(

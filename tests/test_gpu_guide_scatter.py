@@ -71,3 +71,38 @@ def test_slices_add_up(ks, device):
         print("relative L2 difference", err, flush=True)
         assert err < 4e-4
     g.close()
+
+
+@pytest.mark.parametrize("res", [15, 16, 255, 256, 4194303])
+def test_dense_and_hashed_levels(ks, device, res):
+    """Resolutions at which a level stops being dense ((15 + 1)^3 entries are the table's), and whose cube leaves 32 and
+    64 bits ((4194303 + 1)^3 = 2^66). With zero grid features the features' gradient does not depend on the
+    corners' weights, which sum to one: every level of the table holds the same sums as the oracle's, whatever the
+    rounding of a position inside so fine a cell. Bar: that of the gradients."""
+    print("levels", res, flush=True)
+    g = ks.Guide(device, *BOUNDS, ks.guide_config(seed=7, log2_table_size=12, base_resolution=float(res),
+                                                  max_resolution=float(res)))
+    assert g.grid_info()[0].tolist() == [res] * go.LEVELS
+    rng = np.random.default_rng(res % 1000)
+    p = _params(g.n_grid, rng)
+    p[: g.n_grid] = 0
+    g.set_params(p)
+    s = _samples(rng, 1500)
+    _, grad = g.gradient(*s)
+    lay = go.Layout(12, float(res), float(res), *BOUNDS)
+    _, g_ref = go.gradient(p, lay, *s, quantised=True)
+    a, b = (x[: g.n_grid].reshape(go.LEVELS, -1, go.FEATURES).sum(axis=1, dtype=np.float64) for x in (grad, g_ref))
+    assert np.linalg.norm(a - b) < 5e-3 * np.linalg.norm(b)
+    o = g.n_grid
+    assert np.linalg.norm(grad[o:] - g_ref[o:]) < 5e-3 * np.linalg.norm(g_ref[o:])
+    if res < 1000:
+        assert np.linalg.norm(grad[:o] - g_ref[:o]) < 5e-3 * np.linalg.norm(g_ref[:o])
+    assert np.isfinite(g.forward(s[0])).all()
+    g.close()
+
+
+@pytest.mark.parametrize("res", [4294967296.0, float("inf"), float("nan")])
+def test_resolutions_beyond_32_bits_are_refused(ks, device, res):
+    with pytest.raises(ks.KsError) as e:
+        ks.Guide(device, *BOUNDS, ks.guide_config(max_resolution=res))
+    assert e.value.status == ks.KS_ERR_INVALID
