@@ -841,8 +841,19 @@ __global__ __launch_bounds__(kScatterBlock) void k_guide_scatter(GuideNet net, u
     }
 }
 
-// The same with global atomics, one thread per level and position, for tables of so many tiles that going
-// over all positions for each costs more.
+// The same with global atomics, one thread per level and position: 4 us and 13 ns a position at any table size.
+// A tile costs k_guide_scatter its share of clearing and writing 128 KB, and its read of the positions. us with tiles /
+// with atomics, default resolutions (16..256):
+//   table (tiles)    64 samples  2048     8192       32768      262144
+//   2^12 (256)       5 / 5       27 / 31  34 / 118   66 / 488   350 / 4239
+//   2^16 (495)       11 / 5      34 / 32  47 / 122   89 / 508   470 / 4225
+//   2^19 (763)       17 / 5      34 / 36  46 / 135   110 / 550  677 / 4411
+//   2^22 (1722)      38 / 6      64 / 33  88 / 120   209 / 511  1351 / 4281
+//   2^24 (2907)      69 / 6      90 / 33  134 / 125  327 / 526  2236 / 4440
+// The lines cross at about four positions per tile, and never from about 4600 tiles on (a tile's 2.9e-3 ns a position
+// against the 13 ns), which finer grids reach: sixteen hashed levels of 2^22 entries are 4096 tiles.
+constexpr uint32_t kScatterPositionsPerTile = 4;
+constexpr size_t kScatterMaxTiles = 4096;
 __global__ __launch_bounds__(256) void k_guide_scatter_atomic(GuideNet net, uint32_t positions, const float4 *pos,
                                                               const float2 *dx, float *grid_grad) {
     const uint32_t level = blockIdx.y, r = blockIdx.x * 256u + threadIdx.x;
@@ -1086,7 +1097,7 @@ struct ks_guide {
     float lo[3], inv_ext[3];
     DevBuf params, grad, m1, m2, grid_h, w_bf, wt_bf, partials, loss, samples;
     DevBuf rows, pos, dx; // a training slice's input rows, normalised positions and feature gradients
-    DevBuf tiles;         // k_guide_scatter's tiles (n_tiles; 0: the table is scattered with atomics)
+    DevBuf tiles;         // k_guide_scatter's tiles (n_tiles; 0: too many, every batch is scattered with atomics)
     uint32_t n_tiles = 0;
     DevBuf w8, fp8s, act_amax; // FP8 copy of the MLP, its scales, recorded activation maxima
     bool fp8 = false;          // inference in FP8
@@ -1167,8 +1178,8 @@ int launch_extract(const float4 *recs, const float4 *samp, uint32_t n_items, uin
 }
 
 // Loss, weight gradients and grid gradient of n device-resident samples (TrainSample records, every
-// stride-th one) into g->loss and g->grad, whose grid part must be zero (as Adam leaves it). Slices of at most kTrainSlice samples bound the
-// buffers (288 B a sample).
+// stride-th one) into g->loss and g->grad, whose grid part must be zero (as Adam leaves it). Slices of at most
+// kTrainSlice samples bound the buffers (272 B a sample).
 constexpr int64_t kTrainSlice = 1 << 20;
 int gradient_on_device(ks_guide *g, const TrainSample *samples, int64_t n, int stride, float c_scale, float c_max,
                        uint32_t *act_amax, hipStream_t s) {
@@ -1189,7 +1200,7 @@ int gradient_on_device(ks_guide *g, const TrainSample *samples, int64_t n, int s
         hipLaunchKernelGGL(k_guide_train, dim3(waves), dim3(64), kTrainWaveBytes, s, net, m, (uint32_t)stride, chunks,
                            slice, g->rows.as<uint32_t>(), c_scale, c_max, g->dx.as<float2>(), g->partials.as<float>(),
                            g->loss.as<double>(), act_amax);
-        if (g->n_tiles > 0)
+        if (g->n_tiles > 0 && positions >= kScatterPositionsPerTile * g->n_tiles)
             hipLaunchKernelGGL(k_guide_scatter, dim3(g->n_tiles), dim3(kScatterBlock), 0, s, net, positions,
                                g->pos.as<float4>(), g->dx.as<float2>(), g->tiles.as<uint4>(), g->grad.as<float>(), add);
         else
@@ -1303,9 +1314,7 @@ int ks_guide_create(ks_device *dev, const ks_guide_config *cfg_in, const float b
                         tiles.push_back(
                             make_uint4((uint32_t)l, e, std::min(kScatterEntries, used - e), k | (shares << 16)));
             }
-            // A position costs a round of 256 tiles about 0.65 ns and 256 atomics 12 ns: atomics from 16 rounds on
-            // (tables of 2^22 entries and more).
-            if (tiles.size() < 4096) {
+            if (tiles.size() < kScatterMaxTiles) {
                 g->n_tiles = (uint32_t)tiles.size();
                 KS_HIP(g->tiles.alloc(sizeof(uint4) * tiles.size()));
                 KS_HIP(hipMemcpyAsync(g->tiles.p, tiles.data(), sizeof(uint4) * tiles.size(), hipMemcpyHostToDevice,

@@ -1,7 +1,8 @@
 """The grid gradient's accumulation at its edges: batches of one sample, of a wave, of a scatter block and one
-more or less, a batch of more than one slice, and a table whose tiles are so many that it is scattered
-with global atomics. Against the oracle's gradient of the same BF16 operands (bar of test_gpu_guide.py), the
-slices against the sum of their parts."""
+more or less, on both sides of the choice between sums in LDS and global atomics, a batch of more than one slice,
+the largest tables, and a table whose tiles are so many that every batch is scattered with atomics. Against the
+oracle's gradient of the same BF16 operands (bar of test_gpu_guide.py), the slices and the largest tables
+against the sum of their parts."""
 
 import numpy as np
 import pytest
@@ -32,8 +33,10 @@ def _check(g, lay, n, seed):
     assert np.array_equal(grad[:o] != 0, g_ref[:o] != 0)
 
 
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 1023, 1024, 1025])
-@pytest.mark.parametrize("log2_T", [12, 15])  # tiles of one and of several per level, shared over positions
+# tables of 256 tiles and of some 450 (one and several per level, shared over positions): up to four positions a tile
+# are scattered with global atomics, more in LDS
+@pytest.mark.parametrize("log2_T,n", [(12, n) for n in (1, 63, 64, 65, 960, 1023, 1024, 1025, 4097)]
+                         + [(15, n) for n in (1, 63, 64, 65, 1023, 1024, 1025, 1600, 2047, 2049, 4097)])
 def test_batch_edges(ks, device, n, log2_T):
     print("scatter", n, log2_T, flush=True)
     cfg = dict(CONFIGS["small"], log2_table_size=log2_T)
@@ -48,6 +51,39 @@ def test_large_table_uses_atomics(ks, device):
     g = ks.Guide(device, *BOUNDS, ks.guide_config(seed=7, log2_table_size=22, base_resolution=256.0, max_resolution=512.0))
     _check(g, go.Layout(22, 256.0, 512.0, *BOUNDS), 130, 5)
     g.close()
+
+
+def test_large_default_table_in_lds(ks, device):
+    """2^22 entries at the default resolutions: 1722 tiles, in LDS from 6888 positions on."""
+    print("scatter 2^22 in LDS", flush=True)
+    g = ks.Guide(device, *BOUNDS, ks.guide_config(seed=7, log2_table_size=22))
+    _check(g, go.Layout(22, 16.0, 256.0, *BOUNDS), 8192, 6)
+    g.close()
+
+
+@pytest.mark.parametrize("log2_T,tiles", [(23, 2317), (24, 2907)])
+def test_large_default_tables_agree_with_atomics(ks, device, log2_T, tiles):
+    """A batch of more than four positions a tile, scattered in LDS, against its halves, scattered with atomics: the
+    same FP32 terms in another order. An entry of m terms errs by about sqrt(m) 2^-24 of their absolute sum (27 of the
+    coarsest level's, 14 000 of a weight's: 8e-6), with an allowance of 4 for cancellation between them."""
+    print("scatter", log2_T, flush=True)
+    n = 4 * tiles // 64 * 64 + 128
+    g = ks.Guide(device, *BOUNDS, ks.guide_config(seed=7, log2_table_size=log2_T))
+    q, wi, c = _samples(np.random.default_rng(log2_T), n)
+    loss, grad = g.gradient(q, wi, c)
+    k = n // 2
+    l0, want = g.gradient(q[:k], wi[:k], c[:k])
+    l1, part = g.gradient(q[k:], wi[k:], c[k:])
+    g.close()
+    want += part
+    assert loss == pytest.approx(l0 + l1, rel=1e-9)
+    o = len(grad) - go.MLP_SIZE
+    for a, b in ((0, o), (o, o + go.MLP_SIZE)):
+        err = np.linalg.norm(grad[a:b] - want[a:b]) / np.linalg.norm(want[a:b])
+        print("relative L2 difference", err, flush=True)
+        assert err < 3.2e-5
+    # no entry is lost or touched by one of them alone
+    assert np.count_nonzero(grad[:o]) == np.count_nonzero(want[:o])
 
 
 def test_slices_add_up(ks, device):
