@@ -1452,6 +1452,10 @@ struct GuideWork {
     uint32_t stamp = 0; // last record stamp handed out on this device
 };
 
+// Pixels that ks_film_composite takes at a time: a 1080p film at once. The buffer (24 MiB) belongs to the device, so
+// that compositing needs no free device memory, costs a new film nothing more and holds nothing per film.
+constexpr size_t kCompositePixels = 1u << 21;
+
 struct ks_device {
     int ordinal = 0;
     hipStream_t stream = nullptr;
@@ -1467,6 +1471,7 @@ struct ks_device {
     CtrlReport *host_ctrl = nullptr; // pinned, written by k_ctrl_report
     uint8_t *host_scratch = nullptr; // pinned, 64 bytes
     double *relmse_scratch = nullptr; // this device's address of `scratch` (hipGetSymbolAddress at open)
+    DevBuf composite; // kCompositePixels RGB floats for ks_film_composite, allocated at open
     DevBuf perm_tab; // the sampler's permuted digits (kPermTabDims x kPermTabPrefixes words), filled at open
     int sorted_shading = 0;           // material-sorted shading of untextured scenes (ks_device_set_shading)
     uint32_t tail_paths = 0;          // k_tail takes over at or below this many paths (ks_device_set_tail; 0: off)
@@ -1502,7 +1507,6 @@ struct ks_film {
     int32_t w = 0, h = 0;
     float backdrop[3] = {0, 0, 0};
     DevBuf rgb, wts;
-    mutable DevBuf image; // 12 B per pixel for ks_film_composite
 };
 
 struct ks_host_scene {
@@ -2147,6 +2151,7 @@ int ks_device_open(int32_t ordinal, ks_device **out) {
         void *sp = nullptr;
         KS_HIP(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
         d->relmse_scratch = static_cast<double *>(sp);
+        KS_HIP(d->composite.alloc(sizeof(float) * 3 * kCompositePixels));
         KS_HIP(d->perm_tab.alloc(sizeof(uint32_t) * (size_t)kPermTabDims * kPermTabPrefixes));
         hipLaunchKernelGGL(k_perm_tab, dim3(kPermTabDims * kPermTabPrefixes / 256), dim3(256), 0, d->stream,
                            d->perm_tab.as<uint32_t>());
@@ -2991,13 +2996,15 @@ int ks_film_composite(const ks_film *film, float *out) {
         ks_device *dev = film->dev;
         KS_HIP(hipSetDevice(dev->ordinal));
         const size_t n = (size_t)film->w * film->h;
-        DevBuf &img = film->image; // allocated by the film's first composite, kept with the film
-        KS_HIP(img.ensure(sizeof(float) * 3 * n));
-        hipLaunchKernelGGL(k_film_composite, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, dev->stream, n,
-                           film->rgb.as<double>(), film->wts.as<double>(),
-                           make_float3(film->backdrop[0], film->backdrop[1], film->backdrop[2]), img.as<float>());
-        KS_HIP(hipGetLastError());
-        KS_HIP(hipMemcpyAsync(out, img.p, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, dev->stream));
+        float *image = dev->composite.as<float>();
+        for (size_t p = 0; p < n; p += kCompositePixels) {
+            const size_t m = std::min(n - p, kCompositePixels);
+            hipLaunchKernelGGL(k_film_composite, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, dev->stream, m,
+                               film->rgb.as<double>() + 3 * p, film->wts.as<double>() + 2 * p,
+                               make_float3(film->backdrop[0], film->backdrop[1], film->backdrop[2]), image);
+            KS_HIP(hipGetLastError());
+            KS_HIP(hipMemcpyAsync(out + 3 * p, image, sizeof(float) * 3 * m, hipMemcpyDeviceToHost, dev->stream));
+        }
         KS_HIP(hipStreamSynchronize(dev->stream));
         return KS_OK;
     });

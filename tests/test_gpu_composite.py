@@ -2,6 +2,8 @@
 render_target.cpp:187-192, lerp with a float t): equal bit for bit, for films with hits, misses and pixels no
 sample reached, of one pixel, of a block of pixels and one more, and after the film was cleared."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -17,7 +19,8 @@ def expected(rgb, w, backdrop):
         np.float32)
 
 
-@pytest.mark.parametrize("w,h", [(1, 1), (256, 1), (257, 1), (53, 41)])
+# the last two: 2^21 pixels, one part of the device's buffer, and 3073 more
+@pytest.mark.parametrize("w,h", [(1, 1), (256, 1), (257, 1), (53, 41), (2048, 1024), (2049, 1025)])
 @pytest.mark.parametrize("crop", [False, True])
 def test_composite_matches_formula(ks, device, spheres_small, w, h, crop):
     print("composite", w, h, crop, flush=True)
@@ -39,3 +42,22 @@ def test_composite_matches_formula(ks, device, spheres_small, w, h, crop):
         assert np.array_equal(got.view(np.uint32), expected(rgb, wts, backdrop).view(np.uint32))
     film.close()
     sc.close()
+
+
+def test_composite_takes_no_device_memory(ks, device):
+    """A film can be composited however little device memory is free, and holds none for it afterwards."""
+    lib = ks.load_library()
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert lib.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    films = [ks.Film(device, 1920, 1080) for _ in range(4)]
+    before = free()
+    for f in films:
+        f.composite()
+    print("taken by four composites", before - free(), flush=True)
+    assert free() == before
+    for f in films:
+        f.close()
