@@ -1448,6 +1448,7 @@ struct Workspace {
 // records, the extracted training samples and their counter.
 struct GuideWork {
     DevBuf mix, list, recs, train, count;
+    DevBuf scratch; // a training slice's rows, positions and gradients (ksg::device_train_scratch)
     uint32_t mix_q = 0, rec_items = 0;
     uint32_t stamp = 0; // last record stamp handed out on this device
 };
@@ -2108,6 +2109,12 @@ namespace ksg {
 hipStream_t device_stream(ks_device *dev) { return dev->stream; }
 int device_ordinal(ks_device *dev) { return dev->ordinal; }
 int device_cu_count(ks_device *dev) { return dev->n_cu; }
+hipError_t device_train_scratch(ks_device *dev, size_t bytes, uint8_t **out) {
+    hipError_t e = hipSetDevice(dev->ordinal);
+    if (e == hipSuccess) e = dev->gw.scratch.ensure(bytes);
+    *out = dev->gw.scratch.as<uint8_t>();
+    return e;
+}
 } // namespace ksg
 
 // ---------------------------------------------------------------------------------------------------

@@ -1096,7 +1096,6 @@ struct ks_guide {
     uint32_t res[kGuideLevels];
     float lo[3], inv_ext[3];
     DevBuf params, grad, m1, m2, grid_h, w_bf, wt_bf, partials, loss, samples;
-    DevBuf rows, pos, dx; // a training slice's input rows, normalised positions and feature gradients
     DevBuf tiles;         // k_guide_scatter's tiles (n_tiles; 0: too many, every batch is scattered with atomics)
     uint32_t n_tiles = 0;
     DevBuf w8, fp8s, act_amax; // FP8 copy of the MLP, its scales, recorded activation maxima
@@ -1184,6 +1183,14 @@ constexpr int64_t kTrainSlice = 1 << 20;
 int gradient_on_device(ks_guide *g, const TrainSample *samples, int64_t n, int stride, float c_scale, float c_max,
                        uint32_t *act_amax, hipStream_t s) {
     const GuideNet net = net_of(g);
+    // a slice's input rows, normalised positions and feature gradients, the first slice being the largest
+    constexpr size_t kRowBytes = sizeof(uint32_t) * (kGuideIn / 2), kDxBytes = sizeof(float2) * kGuideLevels;
+    const size_t most = ((size_t)std::min(n, kTrainSlice) + 63u) / 64u * 64u;
+    uint8_t *scratch = nullptr;
+    KS_HIP(ksg::device_train_scratch(g->dev, (kRowBytes + sizeof(float4) + kDxBytes) * most, &scratch));
+    uint32_t *rows = reinterpret_cast<uint32_t *>(scratch);
+    float4 *pos = reinterpret_cast<float4 *>(scratch + kRowBytes * most);
+    float2 *dx = reinterpret_cast<float2 *>(scratch + (kRowBytes + sizeof(float4)) * most);
     KS_HIP(hipMemsetAsync(g->loss.p, 0, 3 * sizeof(double), s));
     for (int64_t first = 0; first < n; first += kTrainSlice) {
         const uint32_t m = (uint32_t)std::min<int64_t>(kTrainSlice, n - first), chunks = (m + 63u) / 64u;
@@ -1192,20 +1199,17 @@ int gradient_on_device(ks_guide *g, const TrainSample *samples, int64_t n, int s
         const int add = first > 0 ? 1 : 0;
         const int waves = (int)std::min<uint32_t>(chunks, (uint32_t)std::max(1, ksg::device_cu_count(g->dev) * 3));
         KS_HIP(g->partials.ensure(sizeof(float) * (size_t)waves * kMlpParams));
-        KS_HIP(g->rows.ensure(sizeof(uint32_t) * (kGuideIn / 2) * (size_t)positions));
-        KS_HIP(g->pos.ensure(sizeof(float4) * (size_t)positions));
-        KS_HIP(g->dx.ensure(sizeof(float2) * kGuideLevels * (size_t)positions));
         hipLaunchKernelGGL(k_guide_encode, dim3(positions * kGuideLevels / 256u), dim3(256), 0, s, net, m, (uint32_t)stride,
-                           chunks, slice, g->rows.as<uint32_t>(), g->pos.as<float4>());
+                           chunks, slice, rows, pos);
         hipLaunchKernelGGL(k_guide_train, dim3(waves), dim3(64), kTrainWaveBytes, s, net, m, (uint32_t)stride, chunks,
-                           slice, g->rows.as<uint32_t>(), c_scale, c_max, g->dx.as<float2>(), g->partials.as<float>(),
+                           slice, rows, c_scale, c_max, dx, g->partials.as<float>(),
                            g->loss.as<double>(), act_amax);
         if (g->n_tiles > 0 && positions >= kScatterPositionsPerTile * g->n_tiles)
             hipLaunchKernelGGL(k_guide_scatter, dim3(g->n_tiles), dim3(kScatterBlock), 0, s, net, positions,
-                               g->pos.as<float4>(), g->dx.as<float2>(), g->tiles.as<uint4>(), g->grad.as<float>(), add);
+                               pos, dx, g->tiles.as<uint4>(), g->grad.as<float>(), add);
         else
             hipLaunchKernelGGL(k_guide_scatter_atomic, dim3((positions + 255u) / 256u, kGuideLevels), dim3(256), 0, s, net,
-                               positions, g->pos.as<float4>(), g->dx.as<float2>(), g->grad.as<float>());
+                               positions, pos, dx, g->grad.as<float>());
         hipLaunchKernelGGL(k_guide_reduce, dim3((kMlpParams + 15) / 16), dim3(256), 0, s, g->partials.as<float>(), waves,
                            g->grad.as<float>() + g->n_grid, add);
         KS_HIP(hipGetLastError());

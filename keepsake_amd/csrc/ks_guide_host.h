@@ -17,6 +17,9 @@ namespace ksg {
 hipStream_t device_stream(ks_device *dev);
 int device_ordinal(ks_device *dev);
 int device_cu_count(ks_device *dev);
+// Device memory for one training step's slices, shared by the guides of a device handle (their steps run on its
+// stream, in order) and kept until the handle is closed; grown to `bytes` where it is smaller.
+hipError_t device_train_scratch(ks_device *dev, size_t bytes, uint8_t **out);
 
 constexpr size_t kTrainSampleBytes = 64; // position + weight, normal, wo, wi (4 x float4)
 

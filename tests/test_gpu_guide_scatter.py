@@ -4,6 +4,8 @@ the largest tables, and a table whose tiles are so many that every batch is scat
 oracle's gradient of the same BF16 operands (bar of test_gpu_guide.py), the slices and the largest tables
 against the sum of their parts."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -142,3 +144,33 @@ def test_resolutions_beyond_32_bits_are_refused(ks, device, res):
     with pytest.raises(ks.KsError) as e:
         ks.Guide(device, *BOUNDS, ks.guide_config(max_resolution=res))
     assert e.value.status == ks.KS_ERR_INVALID
+
+
+def test_guides_share_the_training_scratch(ks, device):
+    """A second guide's first step takes memory for its samples (64 B each) and weight partials (768 waves x 11264
+    floats) alone: the rows, positions and gradients between the kernels lie in the device's scratch. Steps by turns
+    give what each guide's own steps give."""
+    lib = ks.load_library()
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert lib.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    n = 1 << 18
+    rng = np.random.default_rng(4)
+    s = [_samples(rng, m) for m in (n, 5000)]
+    g = [ks.Guide(device, *BOUNDS, ks.guide_config(seed=k, **CONFIGS["small"])) for k in (1, 2)]
+    alone = [x.gradient(*b) for x in g[:1] for b in s]
+    before = free()
+    turns = []
+    for b in s:
+        turns.append((g[1].gradient(*b), g[0].gradient(*b)))
+    took = before - free()
+    print("the second guide took", took, flush=True)
+    assert took < 64 * n + 4 * 768 * 11264 + (8 << 20)
+    for (l0, g0), (_, (l1, g1)) in zip(alone, turns):
+        assert l0 == pytest.approx(l1, rel=1e-9)
+        assert np.linalg.norm(g0 - g1) < 1e-4 * np.linalg.norm(g0)
+    for x in g:
+        x.close()
