@@ -148,14 +148,22 @@ constexpr uint32_t kPermTabDims = 128;
 constexpr uint32_t kPermTabPrefixes = 1u << 20;
 constexpr int kPermTabDigits = 10;
 
-KS_DEV uint32_t perm_tab_entry(uint32_t dim, uint32_t p) {
+// The 16 entries of the prefixes 16 h .. 16 h + 15, which share all digits but their lowest two: 29 hashes instead of
+// the 11 of each (the fill is bound by them).
+KS_DEV void perm_tab_group(uint32_t dim, uint32_t h, uint32_t entry[16]) {
     const uint32_t dmask = 0x55555555u * dim;
-    uint32_t e = perm4_of(p ^ dmask) << (2 * kPermTabDigits);
-    for (int k = 0; k < kPermTabDigits; ++k) {
-        const uint32_t digit = (p >> (2 * k)) & 3u;
-        e |= ((perm4_of((p >> (2 * k + 2)) ^ dmask) >> (2 * digit)) & 3u) << (2 * k);
+    uint32_t high = 0u;
+    for (int k = 2; k < kPermTabDigits; ++k)
+        high |= ((perm4_of((h >> (2 * k - 2)) ^ dmask) >> (2 * ((h >> (2 * k - 4)) & 3u))) & 3u) << (2 * k);
+    const uint32_t second = perm4_of(h ^ dmask);
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) {
+        const uint32_t lowest = perm4_of((4u * h + c) ^ dmask), above = high | ((second >> (2 * c)) & 3u) << 2;
+#pragma unroll
+        for (uint32_t d = 0; d < 4; ++d)
+            entry[4 * c + d] = perm4_of((16u * h + 4u * c + d) ^ dmask) << (2 * kPermTabDigits) | above |
+                               ((lowest >> (2 * d)) & 3u);
     }
-    return e;
 }
 
 struct Sobol {
