@@ -54,26 +54,33 @@ def test_batch_equals_single_views(ks, device, cornell, mode):
     sc.close()
 
 
-@pytest.mark.parametrize("graph", [True, False])
-def test_views_split_across_chunks(ks, device, cornell, graph):
+@pytest.mark.parametrize("graph,queue,scale", [(True, 0, 4), (True, 1 << 13, 1), (True, 0, 1), (False, 1 << 13, 1)])
+def test_views_split_across_chunks(ks, device, cornell, graph, queue, scale):
     """A small chunk budget (50 000 items) splits the batch into four chunks, and the spp of the first
     three views across chunk boundaries (segments starting at s0 > 0, one sentinel per chunk): every film
-    still equals its single render bit for bit. The autotuner's probe runs on the first chunk's partial
-    segment list."""
+    still equals its single render bit for bit. At four times the samples and the budget the chunks exceed 2^16 items
+    and the autotuner's probe runs on the first chunk's partial segment list; with a queue smaller than them
+    the chunks are replayed graphs or eager launches; else each is carried out by one thread per path."""
     sc = ks.Scene(device, cornell)
     cam2 = dict(cornell.camera)
     cam2["pos"] = (0.3, 0.4, 2.2)
     specs = [(cornell.camera, dict(render_width=64, render_height=64, spp=16, rng_seed=1)),
              (cam2, dict(render_width=32, render_height=32, spp=64, rng_seed=2)),
              (cornell.camera, dict(render_width=48, render_height=40, spp=9, rng_seed=3))]
+    for _, kw in specs:
+        kw["spp"] *= scale
     views = [(cam, ks.small_pt_params(bounces=12, spp_prog_interval=kw["spp"], **kw), kw) for cam, kw in specs]
     films = [ks.Film(device, kw["render_width"], kw["render_height"]) for _, _, kw in views]
-    kwargs = dict(max_chunk_items=50_000, graph=graph)
-    if not graph:
-        kwargs.update(queue_size=1 << 13, trace_blocks_per_cu=4)
+    kwargs = dict(max_chunk_items=50_000 * scale, graph=graph)
+    if queue:
+        kwargs.update(queue_size=queue, trace_blocks_per_cu=4)
     st = ks.small_pt_render_batch(sc, [(c, p, f) for (c, p, _), f in zip(views, films)], **kwargs)
-    print("chunks", st["batch_chunks"], "queue", st["queue_size"], flush=True)
-    assert st["batch_chunks"] == 4
+    print("chunks", st["batch_chunks"], "queue", st["queue_size"], "iterations", st["iterations"], flush=True)
+    assert st["batch_chunks"] == (4 if scale == 1 else 3)
+    if queue or scale > 1:
+        assert st["iterations"] >= 8 * st["batch_chunks"]
+    else:
+        assert st["iterations"] == 4
     for (cam, p, kw), f in zip(views, films):
         alone = ks.Film(device, kw["render_width"], kw["render_height"])
         ks.small_pt_render(sc, cam, p, alone)

@@ -1,6 +1,7 @@
 """The wavefront loop's end: known from the bounce count where the queue holds the whole pass, read from the
 control block otherwise, and a batch that leaves graph replay for bounded launches. Every path must be
-carried to its end in each, so the films are equal bit for bit."""
+carried to its end in each, so the films are equal bit for bit. Passes of at most 2^16 paths that fit their queue
+are carried out by one thread per path instead, so only the largest size here has a known end."""
 
 import numpy as np
 import pytest
@@ -9,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("bounces", [0, 1, 2, 7, 8, 17])
-@pytest.mark.parametrize("size,spp", [((3, 1), 1), ((31, 17), 3), ((64, 48), 4)])
+@pytest.mark.parametrize("size,spp", [((3, 1), 1), ((31, 17), 3), ((64, 48), 4), ((331, 199), 1)])
 def test_known_and_read_ends_agree(ks, device, cornell, bounces, size, spp):
     print("loop end", bounces, size, spp, flush=True)
     sc = ks.Scene(device, cornell)
@@ -26,6 +27,13 @@ def test_known_and_read_ends_agree(ks, device, cornell, bounces, size, spp):
         else:
             st = ks.small_pt_render(sc, cornell.camera, p, film)
         out.append((film.download(), st["rays_closest"], st["rays_shadow"]))
+        n = w * h * spp
+        if n <= 1 << 16 and n <= max(queue, 256 if queue else n):
+            assert st["iterations"] == 1  # one thread per path
+        elif queue == 0:  # known end: one iteration per vertex of the longest path, unless a read found none left
+            assert st["iterations"] == bounces + 1 or (bounces > 8 and 8 < st["iterations"] <= bounces)
+        else:
+            assert st["iterations"] >= n // queue + bool(n % queue)
         film.close()
     sc.close()
     (rgb, wts), rc, rs = out[0]
