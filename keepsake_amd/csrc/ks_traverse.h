@@ -457,9 +457,9 @@ KS_DEV void trace_rays_kind(const float4 *__restrict__ nodes, const float4 *__re
                 if (st.sp == 0) exhausted = true;
                 else node = st.pop();
             }
-            // leave for the leaf tests when no lane is left without a leaf, or, so that finished lanes
-            // take new rays sooner, when fewer than kTraverseBusyMin lanes are still looking for one while
-            // some lane has finished its ray
+            // leave for the leaf tests when no lane is left without a leaf, or when fewer than kTraverseBusyMin
+            // lanes are still looking for one while some lane has nothing left to visit: its ray ends with its
+            // leaf tests (and with REPLACE the lane takes its next one)
             const uint64_t busy = __ballot(!finished && leaf == 0 && !exhausted);
             if (busy == 0) break;
             if (__popcll(busy) < kTraverseBusyMin && __any(exhausted)) break;
