@@ -289,7 +289,7 @@ int ks_device_set_shading(ks_device *dev, int32_t sorted);
  * cost less than the tail kernel (40.5 against 42.0 ms for a 1080p 64-spp render). While off, plain and
  * batched renders of at most 2^16 paths of untextured scenes, whose paths all fit the queue, are carried out by
  * that kernel as a whole (their rays count as the wavefront's, and queue size and traversal blocks do not
- * matter). Any other value, even 1, and sorted shading send small renders through the wavefront. */
+ * matter), in scenes of 2^19 triangles and more only where the bounces are enough for their number of paths. Any other value, even 1, and sorted shading send small renders through the wavefront. */
 int ks_device_set_tail(ks_device *dev, int32_t max_paths);
 
 /* ---- scene: replaces create_scene + Scene::create_rtc_scene (rtcCommitScene, scene.cpp:144-160),

@@ -1798,6 +1798,7 @@ struct WavefrontOpts {
     bool graph = false;
     int blocks_per_cu = kMaxTraceBlocksPerCu;
     bool whole_paths = true; // a small run may be carried out by one thread per path (runs_whole_paths)
+    uint32_t samples_per_pixel = 1; // of a batched chunk, on average
     // ray capture (eager launches only): every closest-hit and shadow ray of the run, appended as
     // (o, tmin), (d, tmax) pairs to cap_c / cap_s up to cap_max each; cap_n[0], cap_n[1] count them
     float4 *cap_c = nullptr, *cap_s = nullptr;
@@ -1825,21 +1826,33 @@ __global__ void k_capture_done(Queue q, uint32_t shadow, uint32_t *count, uint32
 
 // Renders of at most this many paths (untextured scenes) are carried out by one thread per path: an iteration of
 // so few rays costs the wavefront its slowest ray and its launches, and every path waits for both at each vertex.
-// With more paths the kernel's 3 waves per SIMD hold lanes of ended paths while the wavefront's stay full, and a
-// sky map lit scene is the first to lose. ms, wavefront / whole paths: Cornell 4096 paths 0.51 / 0.37, 65536 0.52 /
-// 0.36, 262144 0.61 / 0.67; room 12288 1.86 / 1.02, 61440 2.00 / 1.15, 262144 2.38 / 2.07; spheres 30000 1.89 /
-// 1.11, 65536 2.25 / 1.64; sky map 65536 1.55 / 1.49, 131072 1.57 / 1.69, 180000 1.62 / 1.81.
+// With more paths the kernel's 3 waves per SIMD hold lanes of ended paths while the wavefront's stay full. ms,
+// wavefront / whole paths, 16 bounces: Cornell 4096 paths 0.51 / 0.37, 65536 0.52 / 0.36, 262144 0.61 / 0.67; room
+// 12288 1.86 / 1.02, 61440 2.00 / 1.15, 262144 2.38 / 2.07.
 constexpr uint64_t kWholePathLimit = 1u << 16;
+// In large scenes, whose rays differ most, a thread has to save enough iterations to make up for the lanes that wait in
+// the traversals of each vertex; those of many samples of a pixel, which the wavefront's full waves trace
+// together, cost it more. Bounces that pay, wavefront / whole paths of 1.31 M triangles (10 M), from crossings measured
+// at 1024 to 65536 paths of 1 to 64 samples a pixel and 0 to 16 bounces: 65536 paths of 1 sample from 4 (7), of 16
+// from 9 (13); 32768 from 3 (5) and 6 (8); 8192 from 2 (3). 65536 paths, 16 samples a pixel, 4 bounces: 1.14 / 1.35
+// ms (2.24 / 3.16); 12 bounces: 2.50 / 2.26. Scenes below 2^19 triangles gain from one bounce on (room, 202 K triangles,
+// 65536 paths of 1 sample: 1 bounce 1.09 times, 4 bounces 1.31, 16 bounces 1.84).
+constexpr int64_t kWholePathsPerBounce = 49152;
 
 // Whether a run of `total` paths through a queue of Q is carried out by one thread per path, in blocks of 64, one
 // wave to a CU as long as there are CUs. Each block needs a row of the statistics; its lanes then have their
 // overflow stacks too, as the overflow area holds kTraceBlock lanes for each row. Sorted shading has kernels of
 // its own (their rounding differs in a few GGX terms), so a sorted render keeps to them whatever its chunks' sizes.
-bool runs_whole_paths(const ks_scene *sc, uint64_t total, uint32_t Q, bool guided, const WavefrontOpts &wo) {
+bool runs_whole_paths(const ks_scene *sc, uint64_t total, uint32_t Q, uint32_t samples_per_pixel, int bounces,
+                      bool guided, const WavefrontOpts &wo) {
     const ks_device *dev = sc->dev;
-    return wo.whole_paths && total <= kWholePathLimit && total <= (uint64_t)Q &&
-           (total + 63) / 64 <= stat_partial_rows(dev) && dev->tail_paths == 0 && !dev->sorted_shading && !guided &&
-           !wo.cap_n && !sc->ds.textured && !sc->ds.alpha;
+    if (!wo.whole_paths || total > kWholePathLimit || total > (uint64_t)Q || (total + 63) / 64 > stat_partial_rows(dev) ||
+        dev->tail_paths != 0 || dev->sorted_shading || guided || wo.cap_n || sc->ds.textured || sc->ds.alpha)
+        return false;
+    int64_t doublings = 0; // of 2^18 triangles
+    for (uint32_t n = sc->info.n_tris >> 19; n > 0; n >>= 1) ++doublings;
+    return doublings == 0 ||
+           kWholePathsPerBounce * (bounces - 1) >= doublings * (int64_t)total * std::min<uint32_t>(samples_per_pixel, 2u);
 }
 
 int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int max_bounces, Timer &tm,
@@ -1869,7 +1882,8 @@ int run_wavefront(ks_scene *sc, RenderConsts rc, uint64_t total, uint32_t Q, int
     };
     const bool graph = wo.graph && !gp;
     // A small render is two launches: ray generation, and one thread per path to its end.
-    if (runs_whole_paths(sc, total, Q, gp != nullptr, wo)) {
+    const uint32_t samples_per_pixel = wo.batch ? wo.samples_per_pixel : (uint32_t)rc.nb;
+    if (runs_whole_paths(sc, total, Q, samples_per_pixel, max_bounces, gp != nullptr, wo)) {
         const unsigned whole_blocks = (unsigned)((total + 63) / 64);
         hipEvent_t e = graph ? nullptr : tm.begin(KS_K_RAYGEN);
         if (wo.batch) hipLaunchKernelGGL(k_raygen<true>, dim3(gen_blocks), dim3(256), 0, s, rc, pb[0], view(0));
@@ -3294,6 +3308,7 @@ struct BatchChunk {
     std::vector<uint32_t> thread_base, seg_items;
     uint64_t items = 0;
     uint32_t threads = 0;
+    uint32_t samples_per_pixel() const { return (uint32_t)(items / std::max(threads, 1u)); }
 };
 
 std::vector<BatchChunk> schedule_batch(const std::vector<RenderConsts> &views, const std::vector<int> &spp,
@@ -3381,7 +3396,9 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
         if (o.queue_size > 0) {
             Q = (uint32_t)std::min<int64_t>(o.queue_size, 1 << 26);
             wo.blocks_per_cu = o.trace_blocks_per_cu > 0 ? o.trace_blocks_per_cu : kMaxTraceBlocksPerCu;
-        } else if (runs_whole_paths(scene, max_items, small_q, false, wo)) {
+        } else if (std::all_of(chunks.begin(), chunks.end(), [&](const BatchChunk &c) {
+                       return runs_whole_paths(scene, c.items, small_q, c.samples_per_pixel(), max_bounces, false, wo);
+                   })) {
             Q = small_q;
         } else if (dev->tune_scene == scene && dev->tune_items == paths) {
             Q = dev->tune_q;
@@ -3457,6 +3474,7 @@ int ks_small_pt_render_batch(ks_scene *scene, int32_t n_views, const ks_batch_vi
             rc.views = dviews.p();
             rc.segs = dsegs.p();
             rc.n_segs = (int32_t)c.segs.size();
+            wo.samples_per_pixel = c.samples_per_pixel();
             e = run_wavefront(scene, rc, c.items, Q, max_bounces, tm, stats, nullptr, wo);
             if (e) return e;
             hipEvent_t ev = tm.begin(KS_K_FILM);

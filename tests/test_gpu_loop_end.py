@@ -65,3 +65,31 @@ def test_whole_paths_equal_the_wavefront(ks, device, name, seed, w, h, spp):
     assert np.array_equal(a, b) and np.array_equal(wa, wb)
     for k in ("rays_closest", "rays_shadow", "rays_tail", "paths", "nonfinite"):
         assert sa[k] == sb[k], k
+
+
+@pytest.mark.parametrize("w,h,spp,bounces,whole", [(128, 128, 1, 2, True), (256, 128, 1, 2, False), (64, 64, 16, 7, True),
+                                                   (64, 64, 16, 6, False), (32, 32, 1, 1, False), (9, 7, 1, 2, True)])
+def test_large_scenes_take_whole_paths_where_bounces_pay(ks, device, w, h, spp, bounces, whole):
+    """1.31 M triangles, 2 doublings of 2^18: 49152 (bounces - 1) against twice the paths, those of several samples a
+    pixel counted double. Either way, and in a batch, the film is that of a queue too small for whole paths."""
+    print("bounces that pay", w, h, spp, bounces, flush=True)
+    hs = ks.procedural_scene("spheres", 1)
+    sc = ks.Scene(device, hs, bvh={"builder": 1})
+    cam = dict(hs.camera)
+    cam["aspect"] = w / h
+    out = []
+    for queue, batch in ((0, False), (max(256, w * h * spp - 1), False), (0, True)):
+        film = ks.Film(device, w, h)
+        p = ks.small_pt_params(bounces=bounces, render_width=w, render_height=h, spp=spp, spp_prog_interval=spp,
+                               queue_size=queue)
+        if batch:
+            st = ks.small_pt_render_batch(sc, [(cam, p, film)])
+        else:
+            st = ks.small_pt_render(sc, cam, p, film)
+        out.append((film.download(), st))
+        film.close()
+    sc.close()
+    for (rgb, wts), st in out[::2]:
+        assert (st["launches"]["tail"] == 1) == whole
+        assert np.array_equal(rgb, out[1][0][0]) and np.array_equal(wts, out[1][0][1])
+        assert st["rays_closest"] == out[1][1]["rays_closest"] and st["rays_shadow"] == out[1][1]["rays_shadow"]
